@@ -29,7 +29,7 @@ size_t net_packs_bytes();
 hipError_t net_forward(const float *x, float *y, void *acts, const void *packs, const float *P,
                        long long n, int grid, hipStream_t s);
 hipError_t net_backward(const float *x, const void *acts, const float *gout, float *gP,
-                        const void *packs, long long n, int grid, hipStream_t s);
+                        const void *packs, long long n, int cus, hipStream_t s);
 int net_forward_grid(long long n, int cus);
 hipError_t net_warm(const FrameDev *frames, int n_frames, long long total, float *u0,
                     const void *packs, const float *P, int grid, hipStream_t s);
@@ -1051,8 +1051,7 @@ extern "C" int ncs_hip_net_backward(ncs_ctx *ctx, const float *params, const flo
   const float *P;
   int rc = packs_for(ctx, params, s, &packs, &P);
   if (rc) return rc;
-  int grid = (int)std::max<long long>(1, std::min<long long>(n, (long long)ctx->cus * 4));
-  HIPCHK(net_backward(x, acts, grad_out, grad_params, packs, n, grid, s));
+  HIPCHK(net_backward(x, acts, grad_out, grad_params, packs, n, ctx->cus, s));
   return NCS_OK;
 }
 

@@ -20,8 +20,9 @@
 // per workgroup, and per wave the input grid / layer 4's partial sums.
 //
 // Backward: the data gradient is the same convolution with flipped,
-// transposed weight packs; the weight gradient is a GEMM over pixels
-// (MFMA with gathered operands), accumulated into FP32 with atomics.
+// transposed weight packs; the weight gradient is a GEMM over pixels whose
+// operands come from transposing LDS reads, kept in registers over all of a
+// workgroup's tiles and added to memory once.
 #include <algorithm>
 
 #include "ncs_common.h"
@@ -142,69 +143,6 @@ __device__ __forceinline__ f4 bias4(const float *bias, int b, int lane) {
 constexpr int kRowShr1 = 0x111;  // lane x <- lane x-1 in its row (0 at x = 0)
 constexpr int kRowShl1 = 0x101;  // lane x <- lane x+1 in its row (0 at x = 15)
 
-// Row y' of a [256][32] BF16 LDS activation buffer as a B operand
-// (lane (g, x): channels 8g..8g+7 of pixel (y', x)); zero outside the tile.
-__device__ __forceinline__ i4 load_row(const __bf16 *buf, int yy, int lane) {
-  i4 z = {0, 0, 0, 0};
-  if (yy < 0 || yy > 15) return z;
-  const int x = lane & 15, g = lane >> 4;
-  return *reinterpret_cast<const i4 *>(buf + ((yy * 16 + x) * kCh + 8 * g));
-}
-
-__device__ __forceinline__ void store4(__bf16 *buf, int y, int lane, int blk, f4 v) {
-  const int x = lane & 15, g = lane >> 4;
-  bf16x4 h;
-  h.x = (__bf16)v.x;
-  h.y = (__bf16)v.y;
-  h.z = (__bf16)v.z;
-  h.w = (__bf16)v.w;
-  *reinterpret_cast<bf16x4 *>(buf + ((y * 16 + x) * kCh + 16 * blk + 4 * g)) = h;
-}
-
-__device__ __forceinline__ f4 load4(const __bf16 *buf, int y, int lane, int blk) {
-  const int x = lane & 15, g = lane >> 4;
-  bf16x4 h = *reinterpret_cast<const bf16x4 *>(buf + ((y * 16 + x) * kCh + 16 * blk + 4 * g));
-  f4 r = {(float)h.x, (float)h.y, (float)h.z, (float)h.w};
-  return r;
-}
-
-// One 32 -> 16*NB channel layer over a tile: out rows via fn(y, blk, acc).
-// A operands: packs + (blk * 9 + tap); B: rows of `in`.
-template <int NB, class Epi>
-__device__ __forceinline__ void conv32(const __bf16 *in, const i4 *__restrict__ packs,
-                                       int lane, Epi epi) {
-  i4 A[NB][9];
-#pragma unroll
-  for (int b = 0; b < NB; b++)
-#pragma unroll
-    for (int t = 0; t < 9; t++) A[b][t] = packs[(b * 9 + t) * 64 + lane];
-  i4 rm = {0, 0, 0, 0};
-  i4 r0 = load_row(in, 0, lane);
-  for (int y = 0; y < 16; y++) {
-    const i4 rp = load_row(in, y + 1, lane);
-    f4 acc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) acc[b] = (f4){0.f, 0.f, 0.f, 0.f};
-    const i4 rows[3] = {rm, r0, rp};
-#pragma unroll
-    for (int dy = 0; dy < 3; dy++) {
-      const i4 c = rows[dy];
-      const i4 l = dpp_i4<kRowShr1>(c);
-      const i4 r = dpp_i4<kRowShl1>(c);
-#pragma unroll
-      for (int b = 0; b < NB; b++) {
-        acc[b] = mfma_bf16(A[b][dy * 3 + 0], l, acc[b]);
-        acc[b] = mfma_bf16(A[b][dy * 3 + 1], c, acc[b]);
-        acc[b] = mfma_bf16(A[b][dy * 3 + 2], r, acc[b]);
-      }
-    }
-#pragma unroll
-    for (int b = 0; b < NB; b++) epi(y, b, acc[b]);
-    rm = r0;
-    r0 = rp;
-  }
-}
-
 // Two floats as packed BF16 (round to nearest even), low half first.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f2 __attribute__((ext_vector_type(2)));
@@ -232,6 +170,16 @@ __device__ __forceinline__ i4 relu_row(f4 a0, f4 a1) {
   r.z = relu_pair(a1.x, a1.y);
   r.w = relu_pair(a1.z, a1.w);
   return r;
+}
+
+// A data gradient's four channels of one pixel as BF16, zero where the
+// activations `act` (BF16, the same channels) are not positive.
+typedef int i2v __attribute__((ext_vector_type(2)));
+typedef short s4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ i2v relu_masked(f4 v, i2v act) {
+  const bf16x4 a = __builtin_bit_cast(bf16x4, act);
+  return (i2v){bf16_pair((float)a.x > 0.0f ? v.x : 0.0f, (float)a.y > 0.0f ? v.y : 0.0f),
+               bf16_pair((float)a.z > 0.0f ? v.z : 0.0f, (float)a.w > 0.0f ? v.w : 0.0f)};
 }
 
 // A register row written as row y of a [256][32] BF16 buffer in the
@@ -388,38 +336,6 @@ __device__ __forceinline__ void in_pad_put(float *in_pad, int row, int col, floa
   *reinterpret_cast<float2 *>(in_pad + 2 * ((row + 1) * 18 + col + 1)) = make_float2(x0, x1);
 }
 
-// A layer whose input has NC <= 3 channels (K = tap * NC + c padded to 32),
-// input FP32 in LDS as [NC][256]; 2 output blocks, accumulators starting
-// from `bias` (zero when null).
-template <int NC, class Epi>
-__device__ __forceinline__ void conv_small(const float *in, const i4 *__restrict__ packs,
-                                           int lane, Epi epi, const float *bias = nullptr) {
-  const i4 A0 = packs[lane], A1 = packs[64 + lane];
-  f4 c0 = {0.f, 0.f, 0.f, 0.f}, c1 = c0;
-  if (bias != nullptr) {
-    c0 = bias4(bias, 0, lane);
-    c1 = bias4(bias, 1, lane);
-  }
-  const int x = lane & 15, g = lane >> 4;
-  for (int y = 0; y < 16; y++) {
-    bf16x8 bv;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const int k = 8 * g + e;
-      float v = 0.0f;
-      if (k < 9 * NC) {
-        const int tap = k / NC, ch = k % NC;
-        const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
-        if (yy >= 0 && yy < 16 && xx >= 0 && xx < 16) v = in[ch * 256 + yy * 16 + xx];
-      }
-      bv[e] = (__bf16)v;
-    }
-    const i4 B = __builtin_bit_cast(i4, bv);
-    epi(y, 0, mfma_bf16(A0, B, c0));
-    epi(y, 1, mfma_bf16(A1, B, c1));
-  }
-}
-
 // Normalises one tile held in the solver's lane layout (lane (g, x) has
 // rows 4g + r, column x) into the padded input grid; returns sigma.
 __device__ __forceinline__ void tile_inputs(const float *d_tile_lane, const float *gm_lane,
@@ -472,7 +388,6 @@ constexpr int kFwdPacks = PK_B4 - PK_L1;
 constexpr int kNetIoFloats = 768;  // max(18 * 18 * 2, 16 * 16 * 3)
 constexpr int kNetWaveFloats = kNetIoFloats + 256;
 constexpr int kNetFwdLdsBytes = kFwdPacks * 1024 + 128 * 4 + kNetWaves * kNetWaveFloats * 4;
-constexpr int kNetLdsBytes = 2 * 256 * kCh * 2 + 3 * 256 * 4;  // backward: two buffers, x, dY
 
 // Copies the forward packs and the biases [b1 | b2 | b3 | b4] into LDS.
 __device__ __forceinline__ void stage_forward(const i4 *__restrict__ packs,
@@ -586,155 +501,408 @@ void net_warm_kernel(const FrameDev *__restrict__ frames, int n_frames, long lon
 // backward
 // ---------------------------------------------------------------------------
 
-// dW[co][ci][tap] += sum_p dz[p][co] * act[p + tap][ci] for 32-channel dz / act
-// ([256][32] BF16 LDS), MFMA over pixel chunks of 32 with gathered operands.
-__device__ __forceinline__ void grad_w32(const __bf16 *dz, const __bf16 *act, float *gW,
-                                         int lane) {
-  const int i = lane & 15, g = lane >> 4;
-  for (int tap = 0; tap < 9; tap++) {
-    const int dy = tap / 3 - 1, dx = tap % 3 - 1;
+// The backward pass of one tile is 2 x 72 MFMA per wave and layer for four
+// waves (a team): the weight gradient is a GEMM over the tile's 256 pixels,
+// the data gradient the forward convolution with flipped, transposed weights.
+// What bounds it is the feed of the matrix cores, so the layout is chosen for
+// that:
+//  * activations and data gradients sit in LDS as 18 x 18 pixels of 32 BF16
+//    channels with a zero border, so a tap is a fixed address offset and no
+//    read needs a bounds check;
+//  * the weight gradient wants 8 pixels of one channel per lane where memory
+//    has channels innermost: the transposing LDS read (ds_read_b64_tr_b16:
+//    lane 16 g + i of a group gets elements 0..3 of column i from the 4 x 16
+//    block the group addresses) takes them straight from the same buffer the
+//    convolution reads.  A K chunk of 32 is rows r and r + 8, so the fragment
+//    of an input row serves all three dy taps;
+//  * each wave keeps its quarter of every layer's weight gradient (one
+//    16 x 16 block of all nine taps) in registers over all its tiles; the
+//    19,393 sums go to memory once per workgroup, through LDS, so that the
+//    atomics are contiguous.
+// One workgroup of two teams per CU (142 KB of LDS) walks its tiles, with the
+// next activations loaded into registers while the present ones are used.
+// Per two tiles a CU takes 17.5k cycles, 10.5k of them matrix work (an
+// in-kernel clock: 5.4k per middle layer, 152 MFMA per wave on two waves per
+// SIMD).  With the parameter packing and the clearing of the sums before it,
+// one call on 1024 tiles went from 1264 us to 51 us and on 8000 from 7306 us
+// to 197 us against the kernel before it (one wave per tile, 16-bit LDS
+// gathers for the weight gradient, every tile's sums added in memory).
+constexpr int kBwdTeams = 2;
+constexpr int kPixBytes = 2 * kCh;                 // one pixel's channels
+constexpr int kRowBytes = 18 * kPixBytes;          // one padded row
+constexpr int kActBytes = 18 * kRowBytes;          // one padded tile
+constexpr int kPlaneBytes = 18 * 32;               // [18 rows][16 pixels] BF16, rows padded
+constexpr int kDyPlanes = 9;                       // (split of 3) x (dx of 3)
+constexpr int kXPlanes = 6;                        // (channel of 2) x (dx of 3)
+constexpr int kTeamBytes = 3 * kActBytes + (kDyPlanes + kXPlanes) * kPlaneBytes;
+constexpr int kBwdLdsBytes = kBwdTeams * kTeamBytes;
+static_assert(kBwdLdsBytes >= (N_PARAMS + kBwdTeams * (27 * kCh + 4)) * 4,
+              "the sums are staged in the same LDS");
+static_assert(OFF_B4 - OFF_W4 < kBwdTeams * 256, "one thread per layer-4 parameter");
+static_assert(kTeamBytes % 16 == 0 && kBwdLdsBytes <= 160 * 1024, "LDS of one CU");
+
+typedef __attribute__((address_space(3))) unsigned char LdsByte;
+typedef __attribute__((address_space(3))) s4v LdsS4;
+
+// Byte of a pixel's 16-channel block in its row: padded column c, block b.
+// The two blocks of columns 8..15 are swapped, so that the two lane groups of
+// a transposed read that are eight columns apart use different banks (a row
+// of 64-byte pixels comes back to the same bank every four).
+__device__ __forceinline__ int pix_block(int c, int b) {
+  return c * kPixBytes + 32 * (b ^ ((c >> 3) & 1));
+}
+
+// 8 pixels of one channel (an operand's K chunk): lane (g, i) gets channel i
+// of the 16-channel block a and b point into, pixels 0..3 and 4..7.
+__device__ __forceinline__ i4 tr_frag(const LdsByte *pa, const LdsByte *pb) {
+  const s4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS4 *)pa);
+  const s4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsS4 *)pb);
+  const i2v ai = __builtin_bit_cast(i2v, a), bi = __builtin_bit_cast(i2v, b);
+  return (i4){ai.x, ai.y, bi.x, bi.y};
+}
+
+__device__ __forceinline__ i4 lds_i4(const LdsByte *p) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) i4 *>(p);
+}
+
+// Weight gradient of a 32 -> 32 layer, this wave's 16 x 16 block of the nine
+// taps: w[tap][co][ci] += sum_p dz[p][co] act[p + tap][ci].  dz and act are
+// the padded tiles, oz[j] and oa[dx][j] the lane's offsets of a transposed
+// read of its block in padded row 0 (j: pixels 0..3 or 4..7 of the chunk, dx:
+// the tap's column); chunk r of dz is its rows r and r + 8, and the act
+// fragment of rows r', r' + 8 meets the chunks r' - dy.
+__device__ __forceinline__ void grad_w32(const LdsByte *dz, const int (&oz)[2],
+                                         const LdsByte *act, const int (&oa)[3][2], f4 (&w)[9],
+                                         f4 &bias, bool with_bias) {
+  const int one2 = 0x3f803f80;  // BF16 1.0, twice
+  const i4 ones = {one2, one2, one2, one2};
+  i4 prev = {0, 0, 0, 0}, cur = prev, next = prev;  // dz chunks r' - 1, r', r' + 1
 #pragma unroll
-    for (int bo = 0; bo < 2; bo++)
+  for (int rp = -1; rp <= 8; rp++) {
+    prev = cur;
+    cur = next;
+    if (rp + 1 <= 7) {
+      next = tr_frag(dz + oz[0] + (rp + 2) * kRowBytes, dz + oz[1] + (rp + 2) * kRowBytes);
+      if (with_bias) bias = mfma_bf16(next, ones, bias);
+    }
 #pragma unroll
-      for (int bi = 0; bi < 2; bi++) {
-        f4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int ch = 0; ch < 8; ch++) {  // pixel chunks of 32
-          bf16x8 av, bv;
+    for (int dx = 0; dx < 3; dx++) {
+      const i4 a = tr_frag(act + oa[dx][0] + (rp + 1) * kRowBytes,
+                           act + oa[dx][1] + (rp + 1) * kRowBytes);
+      if (rp + 1 <= 7) w[0 + dx] = mfma_bf16(next, a, w[0 + dx]);             // dy = -1
+      if (rp >= 0 && rp <= 7) w[3 + dx] = mfma_bf16(cur, a, w[3 + dx]);       // dy = 0
+      if (rp >= 1) w[6 + dx] = mfma_bf16(prev, a, w[6 + dx]);                 // dy = +1
+    }
+  }
+}
+
+// Data gradient of a 32-channel layer for this wave's output block and eight
+// rows, masked by the ReLU of the activations there, as BF16 in registers:
+// the convolution of dz with the flipped, transposed weights (packs: the
+// lane's entries of the nine taps, read from L2 at each use: kept in
+// registers over the tiles they spilled), each accumulator from zero.  z points at the lane's pixel of padded
+// row 8 h, act at the lane's four channels of row 8 h's pixels (padded).
+__device__ __forceinline__ void grad_data32(const LdsByte *z, const LdsByte *act,
+                                            const i4 *__restrict__ packs, i2v (&out)[8]) {
+  i4 A[9];
 #pragma unroll
-          for (int e = 0; e < 8; e++) {
-            const int p = ch * 32 + 8 * g + e;
-            av[e] = dz[p * kCh + 16 * bo + i];
-            const int yy = (p >> 4) + dy, xx = (p & 15) + dx;
-            bv[e] = (yy >= 0 && yy < 16 && xx >= 0 && xx < 16)
-                        ? act[(yy * 16 + xx) * kCh + 16 * bi + i]
-                        : (__bf16)0.0f;
-          }
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc, 0, 0, 0);
+  for (int t = 0; t < 9; t++) A[t] = packs[t * 64];
+  i4 C[4], L[4], R[4];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    C[q] = lds_i4(z + q * kRowBytes);
+    L[q] = dpp_i4<kRowShr1>(C[q]);
+    R[q] = dpp_i4<kRowShl1>(C[q]);
+  }
+#pragma unroll
+  for (int y = 0; y < 8; y += 2) {
+#pragma unroll
+    for (int q = 2; q < 4; q++) {
+      C[q] = lds_i4(z + (y + q) * kRowBytes);
+      L[q] = dpp_i4<kRowShr1>(C[q]);
+      R[q] = dpp_i4<kRowShl1>(C[q]);
+    }
+    f4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int dx = 0; dx < 3; dx++) {
+        const i4 in = dx == 0 ? L[q] : (dx == 1 ? C[q] : R[q]);
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+          const int dy = q - o;
+          if (dy < 0 || dy > 2) continue;
+          acc[o] = mfma_bf16(A[dy * 3 + dx], in, acc[o]);
         }
-        // acc: lane (g, i) holds co = 16 bo + 4g + r, ci = 16 bi + i
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          atomicAdd(&gW[((16 * bo + 4 * g + r) * kCh + 16 * bi + i) * 9 + tap], acc[r]);
       }
+#pragma unroll
+    for (int o = 0; o < 2; o++)
+      out[y + o] = relu_masked(
+          acc[o], *reinterpret_cast<const __attribute__((address_space(3))) i2v *>(
+                      act + (y + o) * kRowBytes));
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      C[q] = C[q + 2];
+      L[q] = L[q + 2];
+      R[q] = R[q + 2];
+    }
   }
 }
 
-// d(bias)[co] += sum_p dz[p][co]
-__device__ __forceinline__ void grad_b32(const __bf16 *dz, float *gb, int lane) {
-  if (lane < kCh) {
-    float s = 0.0f;
-    for (int p = 0; p < 256; p++) s += (float)dz[p * kCh + lane];
-    atomicAdd(&gb[lane], s);
+// The pixel's value in the three dx planes of one quantity: plane dx holds
+// v[row][x + dx - 1] at (row, x), zero where that is outside the tile (those
+// entries, like the padding rows, are never written).
+__device__ __forceinline__ void put_planes(LdsByte *planes, int row, int col, short v) {
+#pragma unroll
+  for (int dx = 0; dx < 3; dx++) {
+    const int x = col + 1 - dx;
+    if (x >= 0 && x < 16)
+      *reinterpret_cast<__attribute__((address_space(3))) short *>(
+          planes + dx * kPlaneBytes + (row + 1) * 32 + 2 * x) = v;
   }
 }
 
-// Data gradient of a 32-channel layer output given via packs (flipped,
-// transposed weights), masked by the ReLU of `mask_act` and written in place
-// of it (each lane rewrites exactly the entries it read).
-__device__ __forceinline__ void grad_data32(const __bf16 *dz_next, __bf16 *act_inout,
-                                            const i4 *__restrict__ packs, int lane) {
-  conv32<2>(dz_next, packs, lane, [&](int y, int b, f4 acc) {
-    f4 a = load4(act_inout, y, lane, b);
-    f4 v;
-    v.x = a.x > 0.0f ? acc.x : 0.0f;
-    v.y = a.y > 0.0f ? acc.y : 0.0f;
-    v.z = a.z > 0.0f ? acc.z : 0.0f;
-    v.w = a.w > 0.0f ? acc.w : 0.0f;
-    store4(act_inout, y, lane, b, v);
-  });
-}
-
-__global__ __launch_bounds__(64) void net_bwd_kernel(const float *__restrict__ xin,
-                                                     const __bf16 *__restrict__ acts,
-                                                     const float *__restrict__ gout,
-                                                     float *__restrict__ gP,
-                                                     const i4 *__restrict__ packs,
-                                                     long long n) {
-  extern __shared__ __align__(16) unsigned char lds_raw[];
-  __bf16 *buf0 = reinterpret_cast<__bf16 *>(lds_raw);
-  __bf16 *buf1 = buf0 + 256 * kCh;
-  float *in2 = reinterpret_cast<float *>(buf1 + 256 * kCh);  // x, then dY
-  float *dy4 = in2 + 512;
-  const int lane = threadIdx.x;
+__global__ __launch_bounds__(kBwdTeams * 256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void net_bwd_kernel(const float *__restrict__ xin, const __bf16 *__restrict__ acts,
+                    const float *__restrict__ gout, float *__restrict__ gP,
+                    const i4 *__restrict__ packs, long long n) {
+  __shared__ __align__(16) unsigned char lds_all[kBwdLdsBytes];
+  const int team = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+  const int tid = threadIdx.x & 255, lane = threadIdx.x & 63;
   const int i = lane & 15, g = lane >> 4;
-  auto load_act = [&](__bf16 *dst, int layer, long long t) {
+  const int hi = wave >> 1, lo = wave & 1;
+  for (int k = threadIdx.x; k < kBwdLdsBytes / 16; k += blockDim.x)
+    reinterpret_cast<i4 *>(lds_all)[k] = (i4){0, 0, 0, 0};
+  __syncthreads();
+
+  LdsByte *const base = (LdsByte *)lds_all + team * kTeamBytes;
+  LdsByte *const buf0 = base, *const buf1 = base + kActBytes, *const buf2 = base + 2 * kActBytes;
+  LdsByte *const dyp = base + 3 * kActBytes, *const xp = dyp + kDyPlanes * kPlaneBytes;
+  // lane offsets: of a transposed read of this wave's blocks (dz: hi, act:
+  // lo) in padded row 0 of the lane's chunk, of the lane's pixel as the
+  // convolution reads it, of its four output channels
+  int o_hi[2], o_lo[3][2];
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int row = 8 * (g >> 1) * kRowBytes + 8 * (i & 3), c = 8 * (g & 1) + 4 * j + (i >> 2);
+    o_hi[j] = row + pix_block(c + 1, hi);
+#pragma unroll
+    for (int dx = 0; dx < 3; dx++) o_lo[dx][j] = row + pix_block(c + dx, lo);
+  }
+  const int conv0 = 8 * hi * kRowBytes + pix_block(i + 1, g >> 1) + 16 * (g & 1);
+  const int own0 = (8 * hi + 1) * kRowBytes + pix_block(i + 1, lo) + 8 * g;
+  // planes: chunk r of a plane is rows r and r + 8, eight pixels per lane
+  const int pl0 = (8 * (g >> 1) + 1) * 32 + 16 * (g & 1);
+  // layer 4: A row m = split * 9 + tap is the split's plane moved by -tap
+  const int m4 = 16 * hi + i < 27 ? 16 * hi + i : 0;
+  const int t4 = m4 % 9;
+  const int dy_off = (3 * (m4 / 9) + 2 - t4 % 3) * kPlaneBytes + pl0 + (1 - t4 / 3) * 32;
+  // layer 1: B column n = tap * 2 + ci, then a column of ones for the bias
+  const int n1 = 16 * lo + i;
+  const int t1 = n1 < 18 ? n1 >> 1 : 0;
+  const int x_off = (3 * (n1 & 1) + t1 % 3) * kPlaneBytes + pl0 + (t1 / 3 - 1) * 32;
+
+  const i4 A4 = packs[(PK_B4 + lo) * 64 + lane];
+  f4 w3[9], w2[9], w1 = {0.f, 0.f, 0.f, 0.f}, w4 = w1, b3 = w1, b2 = w1;
+#pragma unroll
+  for (int t = 0; t < 9; t++) w3[t] = w2[t] = w1;
+  float db4 = 0.0f;
+
+  // one activation tile: four 16-byte pieces per thread, in registers on the
+  // way from memory to a buffer
+  typedef i4 Stage[4];
+  Stage st;
+  auto fetch_to = [&](Stage &st, int layer, long long t) {
     const i4 *src = reinterpret_cast<const i4 *>(acts + (((long long)layer * n + t) * 256) * kCh);
-    i4 *d = reinterpret_cast<i4 *>(dst);
-    for (int k = lane; k < 256 * kCh / 8; k += 64) d[k] = src[k];
+#pragma unroll
+    for (int k = 0; k < 4; k++) st[k] = src[k * 256 + tid];
   };
-  for (long long t = blockIdx.x; t < n; t += gridDim.x) {
-    for (int k = lane; k < 256; k += 64) dy4[k] = gout[t * 256 + k];
-    load_act(buf0, 2, t);  // layer-3 activations
-    __syncthreads();
-    // layer 4: dW4[0][ci][tap] = sum_p dy4[p] a3[p + tap][ci]; db4 = sum dy4
-    for (int q = lane; q < 9 * kCh; q += 64) {
-      const int ci = q % kCh, tap = q / kCh, dy = tap / 3 - 1, dx = tap % 3 - 1;
-      float s = 0.0f;
-      for (int p = 0; p < 256; p++) {
-        const int yy = (p >> 4) + dy, xx = (p & 15) + dx;
-        if (yy >= 0 && yy < 16 && xx >= 0 && xx < 16)
-          s += dy4[p] * (float)buf0[(yy * 16 + xx) * kCh + ci];
-      }
-      atomicAdd(&gP[OFF_W4 + ci * 9 + tap], s);
-    }
-    if (lane == 0) {
-      float s = 0.0f;
-      for (int p = 0; p < 256; p++) s += dy4[p];
-      atomicAdd(&gP[OFF_B4], s);
-    }
-    // dz3 = conv(dy4, flipped W4) masked by a3 > 0 -> buf1
-    conv_small<1>(dy4, packs + PK_B4 * 64, lane, [&](int y, int b, f4 acc) {
-      f4 a = load4(buf0, y, lane, b);
-      f4 v;
-      v.x = a.x > 0.0f ? acc.x : 0.0f;
-      v.y = a.y > 0.0f ? acc.y : 0.0f;
-      v.z = a.z > 0.0f ? acc.z : 0.0f;
-      v.w = a.w > 0.0f ? acc.w : 0.0f;
-      store4(buf1, y, lane, b, v);
-    });
-    __syncthreads();
-    load_act(buf0, 1, t);  // layer-2 activations
-    __syncthreads();
-    grad_w32(buf1, buf0, gP + OFF_W3, lane);
-    grad_b32(buf1, gP + OFF_B3, lane);
-    __syncthreads();
-    grad_data32(buf1, buf0, packs + PK_B3 * 64, lane);  // buf0 = dz2
-    __syncthreads();
-    load_act(buf1, 0, t);  // layer-1 activations
-    __syncthreads();
-    grad_w32(buf0, buf1, gP + OFF_W2, lane);
-    grad_b32(buf0, gP + OFF_B2, lane);
-    __syncthreads();
-    grad_data32(buf0, buf1, packs + PK_B2 * 64, lane);  // buf1 = dz1
-    // layer 1: dW1[co][ci][tap] = sum_p dz1[p][co] x[ci][p + tap]; K = pixels
-    for (int k = lane; k < 512; k += 64) in2[k] = xin[t * 512 + k];
-    __syncthreads();
-    for (int tap = 0; tap < 9; tap++) {
-      const int dy = tap / 3 - 1, dx = tap % 3 - 1;
+  auto put_from = [&](const Stage &st, LdsByte *dst) {
 #pragma unroll
-      for (int bo = 0; bo < 2; bo++) {
-        f4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int ch = 0; ch < 8; ch++) {
-          bf16x8 av, bv;
+    for (int k = 0; k < 4; k++) {
+      const int px = 64 * k + (tid >> 2), part = tid & 3;
+      *reinterpret_cast<__attribute__((address_space(3))) i4 *>(
+          dst + ((px >> 4) + 1) * kRowBytes + pix_block((px & 15) + 1, part >> 1) +
+          16 * (part & 1)) = st[k];
+    }
+  };
+  auto fetch = [&](int layer, long long t) { fetch_to(st, layer, t); };
+  auto put = [&](LdsByte *dst) { put_from(st, dst); };
+  auto put_own = [&](LdsByte *dst, const i2v (&v)[8]) {
 #pragma unroll
-          for (int e = 0; e < 8; e++) {
-            const int p = ch * 32 + 8 * g + e;
-            av[e] = buf1[p * kCh + 16 * bo + i];
-            const int yy = (p >> 4) + dy, xx = (p & 15) + dx;
-            bv[e] = (i < 2 && yy >= 0 && yy < 16 && xx >= 0 && xx < 16)
-                        ? (__bf16)in2[i * 256 + yy * 16 + xx]
-                        : (__bf16)0.0f;
-          }
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc, 0, 0, 0);
+    for (int y = 0; y < 8; y++)
+      *reinterpret_cast<__attribute__((address_space(3))) i2v *>(dst + own0 + y * kRowBytes) = v[y];
+  };
+  // dL/dout of the tile as three BF16 splits (their sum is the FP32 value;
+  // a value past BF16's range keeps its first split only)
+  auto put_dy = [&](float v) {
+    db4 += v;
+    const int row = tid >> 4, col = tid & 15;
+    const __bf16 s0 = (__bf16)v;
+    const bool fin = fabsf((float)s0) <= 3.4e38f;
+    const float r1 = fin ? v - (float)s0 : 0.0f;
+    const __bf16 s1 = (__bf16)r1;
+    const __bf16 s2 = (__bf16)(r1 - (float)s1);
+    put_planes(dyp, row, col, __builtin_bit_cast(short, s0));
+    put_planes(dyp + 3 * kPlaneBytes, row, col, __builtin_bit_cast(short, s1));
+    put_planes(dyp + 6 * kPlaneBytes, row, col, __builtin_bit_cast(short, s2));
+  };
+
+  const long long step = (long long)gridDim.x * kBwdTeams;
+  long long t = (long long)blockIdx.x * kBwdTeams + team;
+  // both teams run the iterations of the first (it has at least as many)
+  const long long first = (long long)blockIdx.x * kBwdTeams;
+  const int iters = first < n ? (int)((n - first + step - 1) / step) : 0;
+  if (t < n) {
+    Stage s2, s1;
+    fetch_to(s2, 2, t);
+    fetch_to(s1, 1, t);
+    const float dy = gout[t * 256 + tid];
+    fetch(0, t);
+    put_from(s2, buf0);
+    put_from(s1, buf1);
+    put_dy(dy);
+  }
+  for (int it = 0; it < iters; it++, t += step) {
+    const bool on = t < n, more = t + step < n;  // uniform over the team
+    i2v own[8];
+    __syncthreads();  // a3 in buf0, a2 in buf1, dy planes; a1 on its way
+    if (on) {
+      // layer 4: dW4[tap][ci] = sum_q dy[q - tap] a3[q] per split of dy
+#pragma unroll
+      for (int r = 0; r < 8; r++)
+        w4 = mfma_bf16(lds_i4(dyp + dy_off + r * 32),
+                       tr_frag(buf0 + o_lo[1][0] + (r + 1) * kRowBytes,
+                               buf0 + o_lo[1][1] + (r + 1) * kRowBytes), w4);
+      // dz3 = conv(dy, flipped W4) masked by a3 > 0, K = tap padded to 32
+      const int m0 = g == 0 ? -1 : 0, m1 = g == 1 ? 0xffff : 0;
+      int v[3][3];  // BF16 dy of rows y - 1 .. y + 1 at x - 1 .. x + 1
+      auto dy_row = [&](int yy, int (&o)[3]) {  // yy: padded row; dx by DPP
+        o[1] = *reinterpret_cast<const __attribute__((address_space(3))) unsigned short *>(
+            dyp + kPlaneBytes + yy * 32 + 2 * i);
+        o[0] = __builtin_amdgcn_update_dpp(0, o[1], kRowShr1, 0xF, 0xF, true);
+        o[2] = __builtin_amdgcn_update_dpp(0, o[1], kRowShl1, 0xF, 0xF, true);
+      };
+      dy_row(8 * hi, v[0]);
+      dy_row(8 * hi + 1, v[1]);
+#pragma unroll
+      for (int y = 0; y < 8; y++) {
+        dy_row(8 * hi + y + 2, v[2]);
+        const i4 B = {(m0 & (v[0][0] | v[0][1] << 16)) | (m1 & v[2][2]),
+                      m0 & (v[0][2] | v[1][0] << 16), m0 & (v[1][1] | v[1][2] << 16),
+                      m0 & (v[2][0] | v[2][1] << 16)};
+        const f4 z = {0.f, 0.f, 0.f, 0.f};
+        own[y] = relu_masked(
+            mfma_bf16(A4, B, z), *reinterpret_cast<const __attribute__((address_space(3))) i2v *>(
+                                     buf0 + own0 + y * kRowBytes));
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) {
+          v[0][dx] = v[1][dx];
+          v[1][dx] = v[2][dx];
         }
-        if (i < 2)
-#pragma unroll
-          for (int r = 0; r < 4; r++)
-            atomicAdd(&gP[OFF_W1 + ((16 * bo + 4 * g + r) * 2 + i) * 9 + tap], acc[r]);
       }
     }
-    grad_b32(buf1, gP + OFF_B1, lane);
+    __syncthreads();  // every read of a3 is done
+    float x0 = 0.0f, x1 = 0.0f;
+    if (on) {
+      put_own(buf0, own);
+      put(buf2);
+      x0 = xin[t * 512 + tid];
+      x1 = xin[t * 512 + 256 + tid];
+    }
+    if (more) fetch(2, t + step);
+    __syncthreads();  // dz3 in buf0, a2 in buf1, a1 in buf2
+    if (on) {
+      put_planes(xp, tid >> 4, tid & 15, __builtin_bit_cast(short, (__bf16)x0));
+      put_planes(xp + 3 * kPlaneBytes, tid >> 4, tid & 15, __builtin_bit_cast(short, (__bf16)x1));
+      grad_w32(buf0, o_hi, buf1, o_lo, w3, b3, lo == 0);
+      grad_data32(buf0 + conv0, buf1 + own0, packs + (PK_B3 + lo * 9) * 64 + lane + opaque_zero(), own);
+    }
     __syncthreads();
+    if (on) put_own(buf1, own);
+    if (more) {
+      put(buf0);
+      fetch(1, t + step);
+    }
+    __syncthreads();  // dz2 in buf1, a1 in buf2
+    if (on) {
+      grad_w32(buf1, o_hi, buf2, o_lo, w2, b2, lo == 0);
+      grad_data32(buf1 + conv0, buf2 + own0, packs + (PK_B2 + lo * 9) * 64 + lane + opaque_zero(), own);
+    }
+    __syncthreads();
+    if (on) put_own(buf2, own);
+    if (more) {
+      put(buf1);
+      fetch(0, t + step);
+      put_dy(gout[(t + step) * 256 + tid]);
+    }
+    __syncthreads();  // dz1 in buf2
+    if (on) {
+      const int one2 = 0x3f803f80;
+      const i4 ones = {one2, one2, one2, one2};
+#pragma unroll
+      for (int r0 = 0; r0 < 8; r0 += 4) {
+        i4 za[4], xb[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          za[r] = tr_frag(buf2 + o_hi[0] + (r0 + r + 1) * kRowBytes,
+                          buf2 + o_hi[1] + (r0 + r + 1) * kRowBytes);
+          xb[r] = lds_i4(xp + x_off + (r0 + r) * 32);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) w1 = mfma_bf16(za[r], n1 == 18 ? ones : xb[r], w1);
+      }
+    }
+  }
+
+  // The workgroup's sums, in the order of the parameters in LDS: the first
+  // team stores, the second adds (LDS float atomics took 50 us here), then
+  // one contiguous pass of atomics to memory.  Layer 4's three splits and
+  // the waves' parts of its bias are added up on the way out.
+  __syncthreads();
+  for (int off = 32; off >= 1; off >>= 1) db4 += __shfl_xor(db4, off);
+  float *const sum = reinterpret_cast<float *>(lds_all);
+  float *const sum4 = sum + N_PARAMS;               // [team][27][32]
+  float *const sumb = sum4 + kBwdTeams * 27 * kCh;  // [team][wave]
+  for (int q = 0; q < kBwdTeams; q++) {
+    if (team == q) {
+      auto add = [&](int k, float v) { sum[k] = q == 0 ? v : sum[k] + v; };
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int co = 16 * hi + 4 * g + r;
+        const int k = (co * kCh + 16 * lo + i) * 9;
+#pragma unroll
+        for (int tp = 0; tp < 9; tp++) {
+          add(OFF_W3 + k + tp, w3[tp][r]);
+          add(OFF_W2 + k + tp, w2[tp][r]);
+        }
+        if (lo == 0 && i == 0) {
+          add(OFF_B3 + co, b3[r]);
+          add(OFF_B2 + co, b2[r]);
+        }
+        if (n1 < 18) add(OFF_W1 + (co * 2 + (n1 & 1)) * 9 + (n1 >> 1), w1[r]);
+        if (n1 == 18) add(OFF_B1 + co, w1[r]);
+        const int m = 16 * hi + 4 * g + r;
+        if (m < 27) sum4[(q * 27 + m) * kCh + 16 * lo + i] = w4[r];
+      }
+      if (lane == 0) sumb[q * 4 + wave] = db4;
+    }
+    __syncthreads();
+  }
+  for (int k = threadIdx.x; k < OFF_W4; k += blockDim.x) atomicAdd(&gP[k], sum[k]);
+  if (threadIdx.x < OFF_B4 - OFF_W4) {
+    const int ci = threadIdx.x / 9, tp = threadIdx.x - 9 * ci;
+    float v = 0.0f;
+#pragma unroll
+    for (int m = 0; m < kBwdTeams * 3; m++) v += sum4[(m * 9 + tp) * kCh + ci];
+    atomicAdd(&gP[OFF_W4 + threadIdx.x], v);
+  }
+  if (threadIdx.x == OFF_B4 - OFF_W4) {
+    float v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kBwdTeams * 4; k++) v += sumb[k];
+    atomicAdd(&gP[OFF_B4], v);
   }
 }
 
@@ -780,10 +948,12 @@ hipError_t net_forward(const float *x, float *y, void *acts, const void *packs, 
 }
 
 hipError_t net_backward(const float *x, const void *acts, const float *gout, float *gP,
-                        const void *packs, long long n, int grid, hipStream_t s) {
+                        const void *packs, long long n, int cus, hipStream_t s) {
   hipLaunchKernelGGL(fill_kernel, dim3(64), dim3(256), 0, s, gP, (long long)N_PARAMS, 0.0f);
   if (n <= 0) return hipGetLastError();
-  hipLaunchKernelGGL(net_bwd_kernel, dim3(grid), dim3(64), kNetLdsBytes, s, x,
+  const long long pairs = (n + kBwdTeams - 1) / kBwdTeams;
+  const int grid = (int)std::max<long long>(1, std::min<long long>(pairs, cus));
+  hipLaunchKernelGGL(net_bwd_kernel, dim3(grid), dim3(kBwdTeams * 256), 0, s, x,
                      reinterpret_cast<const __bf16 *>(acts), gout, gP,
                      reinterpret_cast<const i4 *>(packs), n);
   return hipGetLastError();
