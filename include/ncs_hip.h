@@ -98,7 +98,8 @@ typedef struct {
                           per direction, fewer iterations).  0: the scalar
                           s.y/y.y of liblbfgs and ncs.cl:1123 */
   int waves_per_group; /* tiles (waves) per workgroup, 1..4; 0 = autotuned
-                          (else 1) */
+                          (else 4, or 1 for a batch of at most four tiles
+                          per CU) */
   int precision;       /* NCS_PRECISION_* */
 } ncs_params;
 

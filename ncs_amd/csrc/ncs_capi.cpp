@@ -16,7 +16,7 @@
 namespace ncs {
 int solve_waves_per_cu(int m, bool general, bool pad, bool f16, int wpg);
 hipError_t launch_solve(int m, bool general, bool pad, bool f16, unsigned int waves, int wpg,
-                        hipStream_t s, const SolveArgs &a);
+                        hipStream_t s, SolveArgs a);
 hipError_t launch_adu_to_photons(const uint16_t *adu, const float *offset, const float *gain,
                                  float *out, long long n, hipStream_t s);
 hipError_t launch_gamma_from_camera(const float *var, const float *gain, float *gamma,
@@ -96,7 +96,7 @@ struct DevBuf {
 struct Schedule {
   int history = 5;
   int waves_per_cu = 0;  // 0: the occupancy limit
-  int wpg = 1;
+  int wpg = 0;           // 0: default_group()
   bool f16 = false;      // FP16-split basis changes (else FP32)
 };
 
@@ -122,6 +122,9 @@ struct ncs_ctx {
   float k_norm = 0.0f;  // max row sum |2 q_ee| + |2 q_oo| of the mask tables
   // autotuned schedules, keyed by (general mask, padded geometry, FP16 split)
   std::map<TuneKey, Schedule> tuned;
+  // occupancy limits, by history, general mask, padded geometry, FP16 split
+  // and waves per workgroup (0: not asked yet)
+  mutable int waves_per_cu[9][2][2][2][kMaxWavesPerGroup + 1] = {};
   // last uploaded frame descriptors (pinned staging + completion event)
   std::vector<FrameDev> last_frames;
   bool frames_valid = false;
@@ -625,14 +628,34 @@ static bool any_pad(const ncs_ctx *ctx, const ncs_frame *frames, int n) {
   return false;
 }
 
-// The schedule of a solve: explicit params win, then the autotuned schedule
-// of this mask kind and geometry, then history 5, one wave per workgroup and
-// the occupancy limit.
-static Schedule resolve_schedule(const ncs_ctx *ctx, const ncs_params *p, bool pad) {
+// Waves per workgroup without a tuned schedule.  A workgroup shares one copy
+// of the solver's tables in LDS, which beside the histories decides how many
+// waves a CU holds: four per group hold the most at every depth (history 5:
+// 12 against 9 with one; 4 frames of 2048^2 469 against 541 us, 10 frames at
+// history 1 690 against 856 us).  A batch of at most one tile per SIMD leaves
+// the CUs room anyway and starts fastest one wave at a time (30 windows: 16.4
+// against 17.2 us).
+static int default_group(const ncs_ctx *ctx, long long total) {
+  return total <= 4LL * ctx->cus ? 1 : 4;
+}
+
+// Waves of a schedule's kernel one CU holds at once (asked once per kernel).
+static int occupancy(const ncs_ctx *ctx, int history, bool pad, bool f16, int wpg) {
+  int &w = ctx->waves_per_cu[history][ctx->general][pad][f16][wpg];
+  if (w == 0) w = std::max(1, solve_waves_per_cu(history, ctx->general, pad, f16, wpg));
+  return w;
+}
+
+// The schedule of a solve of `total` tiles: explicit params win, then the
+// autotuned schedule of this mask kind and geometry, then history 5,
+// default_group() and the occupancy limit.
+static Schedule resolve_schedule(const ncs_ctx *ctx, const ncs_params *p, bool pad,
+                                 long long total) {
   const bool f16 = p->precision == NCS_PRECISION_F16_SPLIT;
   Schedule d;
   auto it = ctx->tuned.find(TuneKey{ctx->general, pad, f16});
   if (it != ctx->tuned.end()) d = it->second;
+  else d.wpg = default_group(ctx, total);
   Schedule s;
   s.f16 = f16;
   s.history = p->history > 0 ? p->history : d.history;
@@ -640,10 +663,7 @@ static Schedule resolve_schedule(const ncs_ctx *ctx, const ncs_params *p, bool p
   // a tuned grid only applies to the depth and workgroup size it was tuned for
   const bool same = s.history == d.history && s.wpg == d.wpg;
   s.waves_per_cu = p->waves_per_cu > 0 ? p->waves_per_cu : (same ? d.waves_per_cu : 0);
-  if (s.waves_per_cu <= 0) {
-    int w = solve_waves_per_cu(s.history, ctx->general, pad, s.f16, s.wpg);
-    s.waves_per_cu = w > 0 ? w : 8;
-  }
+  if (s.waves_per_cu <= 0) s.waves_per_cu = occupancy(ctx, s.history, pad, s.f16, s.wpg);
   return s;
 }
 
@@ -701,7 +721,7 @@ static int enqueue_solve(ncs_ctx *ctx, const FrameDev *d_frames, int n_frames, b
   if (total <= 0) return NCS_OK;
   SolveArgs a = make_args(ctx, d_frames, n_frames, total, p, u0, u_tiles, iters, status, cost,
                           queue);
-  HIPCHK(launch_schedule(ctx, resolve_schedule(ctx, p, pad), pad, total, s, a));
+  HIPCHK(launch_schedule(ctx, resolve_schedule(ctx, p, pad, total), pad, total, s, a));
   return NCS_OK;
 }
 
@@ -800,7 +820,8 @@ extern "C" int ncs_hip_reduce_frames_device_noalloc(ncs_ctx *ctx, const ncs_fram
     hipLaunchKernelGGL(write_frames_kernel, dim3(1), dim3(64), 0, s, c, dfr);
     HIPCHK(hipGetLastError());
   }
-  // the counters are reset by a kernel before the solve (launch_solve)
+  // the counters, where the launch needs them, are reset by a kernel before
+  // the solve (launch_solve)
   return enqueue_solve(ctx, dfr, n_frames, any_pad(ctx, frames, n_frames), total, params,
                        params->start == NCS_START_TILES ? u0_tiles : nullptr, nullptr,
                        iterations, status, cost, dq, s);
@@ -1168,9 +1189,9 @@ extern "C" int ncs_hip_autotune(ncs_ctx *ctx, const ncs_frame *frames, int n_fra
   const bool f16 = base->precision == NCS_PRECISION_F16_SPLIT;
   Schedule def;
   def.history = base->history > 0 ? base->history : 5;
-  def.wpg = 1;
+  def.wpg = default_group(ctx, total);
   def.f16 = f16;
-  def.waves_per_cu = std::max(1, solve_waves_per_cu(def.history, ctx->general, pad, f16, 1));
+  def.waves_per_cu = occupancy(ctx, def.history, pad, f16, def.wpg);
   float ms_def = 0.0f;
   e = time_one(def, &ms_def);
   struct Cand {
@@ -1187,8 +1208,7 @@ extern "C" int ncs_hip_autotune(ncs_ctx *ctx, const ncs_frame *frames, int n_fra
   for (int m : depths) {
     for (int wpg : groups) {
       if (e != hipSuccess) break;
-      const int occ = solve_waves_per_cu(m, ctx->general, pad, f16, wpg);
-      if (occ <= 0) continue;
+      const int occ = occupancy(ctx, m, pad, f16, wpg);
       std::vector<int> grid = {occ, std::max(wpg, (occ * 3 / 4) / wpg * wpg),
                                std::max(wpg, (occ / 2) / wpg * wpg)};
       std::sort(grid.begin(), grid.end());
@@ -1388,7 +1408,7 @@ extern "C" int ncs_hip_pipeline_create(ncs_ctx *ctx, const ncs_pipeline_frame *f
   pl->gamma_set.assign(n_frames, 0);
   pl->levels.assign(n_frames, 1);
   pl->level_points.resize(n_frames);
-  pl->sched = resolve_schedule(ctx, params, pl->pad);
+  pl->sched = resolve_schedule(ctx, params, pl->pad, pl->total);
   pl->win = ctx->win;
   *out = pl.release();
   return NCS_OK;

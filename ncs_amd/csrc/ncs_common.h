@@ -14,14 +14,11 @@ constexpr int kWave = 64;          // gfx950 wavefront
 constexpr int kWavesPerBlock = 4;  // 256-thread workgroups, one tile per wave
 constexpr int kMaxWavesPerGroup = 4;  // persistent solver: waves per workgroup 1..4
 
-// Work queue of the persistent solver: 7/8 of the tiles are assigned to the
-// waves statically in contiguous blocks; the rest are split into kQueues
-// contiguous ranges, one per XCD (workgroups are dispatched round-robin over
-// the 8 XCDs), each with its own counter on its own 128-byte line, taken
-// kChunk tiles per atomic.
+// Work queue of the persistent solver: kQueues counters, one per XCD
+// (workgroups are dispatched round-robin over the 8 XCDs), each on its own
+// 128-byte line (see TileSchedule).
 constexpr int kQueues = 8;
 constexpr int kQueueStride = 32;   // unsigned ints between counters
-constexpr int kChunk = 4;
 constexpr size_t kQueueBytes = kQueues * kQueueStride * sizeof(unsigned int);
 constexpr float kFitMin = 1.0e-6f; // negative-value guard (ncs.cl:45, ncs.c:169)
 
@@ -60,11 +57,22 @@ struct FrameDev {
   long long slot;      // per-tile array index of the frame's first tile
 };
 
+// How a launch's tiles are shared out.  The first dyn0 tiles are static: the
+// first `extra` waves own per_wave + 1 contiguous tiles each, the others
+// per_wave.  The tiles from dyn0 on form kQueues ranges, one per XCD, that
+// waves take from one by one with an atomic, their home range first, then
+// the next one.
+struct TileSchedule {
+  unsigned int per_wave, extra;
+  unsigned int dyn0;
+};
+
 // Solver parameters in the kernel's units.
 struct SolveArgs {
   const FrameDev *frames;
   int n_frames;
   long long total_tiles;
+  TileSchedule sched;          // filled in by launch_solve
   unsigned int *queue;         // kQueues work-queue counters (kQueueBytes)
   const float *tables;         // [64][16] per-lane OTF/DFT tables
   const float *u0;             // [tiles][256] warm start or nullptr

@@ -653,6 +653,9 @@ __device__ __forceinline__ int mt_post(MtState &S, float &stp, float f, float dg
 // The persistent solver kernel
 // ---------------------------------------------------------------------------
 
+// Dynamic ranges a wave takes tiles from: its home range and the next one.
+constexpr int kScan = 2;
+
 // The frame table seen through the constant address space (scalar loads).
 typedef __attribute__((address_space(4))) const FrameDev FrameConst;
 
@@ -768,6 +771,17 @@ __device__ __forceinline__ void ll_trial(float t, const float (&u)[4], const flo
   wave_sum<2>(red);
 }
 
+// The curvature-corrected H0 is built for histories up to 3; above that its
+// two basis changes per direction cost more than the iterations it saves
+// (measured at history 5), and precond 2 runs as precond 1.
+constexpr int kCorrHistory = 3;
+
+// LDS of one wave, in float4 per lane: the s and y vectors of the history,
+// and the stash of the curvature-corrected H0 where there is one.
+__host__ __device__ constexpr int wave_lds_f4(int m) {
+  return 2 * m + (m <= kCorrHistory ? 1 : 0);
+}
+
 // One to kMaxWavesPerGroup waves per workgroup, each solving its own tiles;
 // a wave's L-BFGS history lives in its slice of LDS as two rings of M vectors,
 // followed by one vector of scratch for the curvature-corrected H0 (each
@@ -800,12 +814,9 @@ void solve_kernel(SolveArgs A) {
   __shared__ MtState mt_state[kMaxWavesPerGroup];  // line-search state per wave
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform
   constexpr bool kCacheIv = M <= 3;  // keep 1/(u+gamma) across iterations
-  // The curvature-corrected H0 is built for histories up to 3; above that its
-  // two basis changes per direction cost more than the iterations it saves
-  // (measured at history 5), and precond 2 runs as precond 1.
-  constexpr bool kCorr = M <= 3;
+  constexpr bool kCorr = M <= kCorrHistory;
   MtState &mt_lds = mt_state[wave];
-  float4 *const Sb = lds_hist + wave * ((2 * M + 1) * 64);  // s vectors, ring of M
+  float4 *const Sb = lds_hist + wave * (wave_lds_f4(M) * 64);  // s vectors, ring of M
   float4 *const Yb = Sb + M * 64;                           // y vectors, ring of M
   float4 *const Hz = Yb + M * 64 + (threadIdx.x & 63);      // this lane's H0 stash
   const int lane = threadIdx.x & 63;
@@ -824,48 +835,34 @@ void solve_kernel(SolveArgs A) {
   const TT T{tab_lds + lane * TT::kCount};
   const auto GB = basis32<F16>(T, A.tables);
 
-  // Tile schedule.  Device-scope atomics are slow on this part (they are
-  // resolved beyond the XCD's L2), so half the tiles are assigned statically:
-  // wave w owns the contiguous block [w S, w S + S), S = floor(total / 2 /
-  // waves).  The rest are split into kQueues ranges, one per XCD, that waves
-  // take kChunk at a time with one atomic per chunk, home range first, then
-  // the others.  Tiles differ in iterations, so the dynamic half is what
-  // balances the waves: a static 7/8 (or 3/4) left the launch 7% (4%) longer,
-  // and a larger dynamic share gained nothing more.  next_tile() gives the wave's next
-  // tile (uniform) or -1 when every range is exhausted.
-  // Tile indices fit 32 bits (the host caps a batch below 2^32 tiles).  The
-  // static block is the wave's first chunk [next, end).
-  const unsigned int total = (unsigned int)A.total_tiles;
+  // next_tile() gives the wave's next tile (uniform) or -1 when its static
+  // block [next, end) and the dynamic ranges it takes from are exhausted
+  // (TileSchedule; launch_solve has the shares).  Tile indices fit 32 bits
+  // (the host caps a batch below 2^32 tiles).  A wave looks into its home
+  // range and one other: an atomic on an exhausted range costs a device-scope
+  // round trip like any other, and with all eight tried the end of the launch
+  // was 30 us longer (one 2048^2 frame: 120 us, 89 us with two).
   unsigned int next, end;
   {
-    const unsigned int n_waves = gridDim.x * (blockDim.x >> 6);
-    const unsigned int per_wave = (total - total / 2) / n_waves;
-    next = (blockIdx.x * (blockDim.x >> 6) + wave) * per_wave;
-    end = next + per_wave;
+    const unsigned int w = blockIdx.x * (blockDim.x >> 6) + wave;
+    next = w * A.sched.per_wave + min(w, A.sched.extra);
+    end = next + A.sched.per_wave + (w < A.sched.extra ? 1u : 0u);
   }
   int qv = 0;  // dynamic ranges found exhausted
   auto next_tile = [&]() -> long long {
-    if (next >= end) {
-      const unsigned int n_waves = gridDim.x * (blockDim.x >> 6);
-      const unsigned int dyn0 = (total - total / 2) / n_waves * n_waves;
-      const unsigned int nd = total - dyn0;
-      while (qv < kQueues) {
-        const int q = (blockIdx.x + qv) % kQueues;  // home range first
-        const unsigned int lo = dyn0 + (unsigned int)((unsigned long long)nd * q / kQueues);
-        const unsigned int hi = dyn0 + (unsigned int)((unsigned long long)nd * (q + 1) / kQueues);
-        unsigned int got = 0;
-        if (lane == 0) got = atomicAdd(A.queue + q * kQueueStride, (unsigned int)kChunk);
-        got = (unsigned int)__builtin_amdgcn_readfirstlane((int)got);
-        if (got < hi - lo) {
-          next = lo + got;
-          end = min(hi, next + (unsigned int)kChunk);
-          break;
-        }
-        qv++;
-      }
-      if (next >= end) return -1;
+    if (next < end) return (long long)(next++);
+    const unsigned int dyn0 = A.sched.dyn0, nd = (unsigned int)A.total_tiles - dyn0;
+    if (nd == 0) return -1;
+    for (; qv < kScan; qv++) {
+      const int q = (blockIdx.x + qv) % kQueues;  // home range first
+      const unsigned int lo = dyn0 + (unsigned int)((unsigned long long)nd * q / kQueues);
+      const unsigned int hi = dyn0 + (unsigned int)((unsigned long long)nd * (q + 1) / kQueues);
+      unsigned int got = 0;
+      if (lane == 0) got = atomicAdd(A.queue + q * kQueueStride, 1u);
+      got = (unsigned int)__builtin_amdgcn_readfirstlane((int)got);
+      if (got < hi - lo) return (long long)(lo + got);
     }
-    return (long long)(next++);
+    return -1;
   };
 
   // The frame table is read through the constant address space (scalar
@@ -1497,6 +1494,9 @@ hipError_t launch_eval(bool general, const float *data, const float *gamma, cons
   return hipGetLastError();
 }
 
+// Half tiles per wave (4.5 tiles) up to which a launch is all static.
+constexpr long long kStaticHalfTiles = 9;
+
 // Resets the work-queue counters (a kernel, not a memset, so that captured
 // graphs replay it correctly).
 __global__ void reset_queue_kernel(unsigned int *q) {
@@ -1533,7 +1533,7 @@ static SolveKernelFn solve_kernel_for(int m, bool general, bool pad, bool f16) {
 }
 
 static size_t solve_lds_bytes(int m, int wpg) {
-  return (size_t)wpg * (2 * m + 1) * 64 * sizeof(float4);
+  return (size_t)wpg * wave_lds_f4(m) * 64 * sizeof(float4);
 }
 
 // Waves of this instantiation one CU holds at once with workgroups of `wpg`
@@ -1549,14 +1549,38 @@ int solve_waves_per_cu(int m, bool general, bool pad, bool f16, int wpg) {
   return blocks * wpg;
 }
 
-// Resets the queue and launches `waves` persistent waves in workgroups of
-// `wpg` waves (waves is rounded up to a multiple of wpg).
+// Launches `waves` persistent waves in workgroups of `wpg` waves (waves is
+// rounded up to a multiple of wpg).
+//
+// Shares of the tiles.  A device-scope atomic is resolved beyond the XCD's
+// L2, so tiles are assigned statically where that balances: up to
+// 4.5 tiles per wave all of them (each SIMD's handful of waves ends
+// with the same number of tiles give or take one, and the launch needs no
+// counters; one tile per wave is the smallest batch's best: 30 windows went
+// from 55 us, in chunks on eight waves, to 16 us).  Above that two fifths,
+// and the rest one by one, which evens out the waves: with history 1 and the
+// linear start, 10 frames of 2048^2 take 704 us at one half static in chunks
+// of four, 671 us as here (664 at one quarter, 722 at four fifths); with
+// history 5 and the plain start 1095 and 1084 us (1087, 1140); one frame
+// 120 and 87 us, 150 and 128 us.  Chunks of two or three were within 1% with
+// the linear start's short tiles and 2% slower with the plain start's.
 hipError_t launch_solve(int m, bool general, bool pad, bool f16, unsigned int waves, int wpg,
-                        hipStream_t s, const SolveArgs &a) {
+                        hipStream_t s, SolveArgs a) {
   SolveKernelFn fn = solve_kernel_for(m, general, pad, f16);
   if (!fn || wpg < 1 || wpg > kMaxWavesPerGroup || waves == 0) return hipErrorInvalidValue;
   const unsigned int groups = (waves + wpg - 1) / wpg;
-  hipLaunchKernelGGL(reset_queue_kernel, dim3(1), dim3(64), 0, s, a.queue);
+  const long long n_waves = (long long)groups * wpg;
+  // (every range needs a workgroup that calls it home)
+  if (2 * a.total_tiles <= kStaticHalfTiles * n_waves || groups < (unsigned int)kQueues) {
+    a.sched.per_wave = (unsigned int)(a.total_tiles / n_waves);
+    a.sched.extra = (unsigned int)(a.total_tiles % n_waves);
+    a.sched.dyn0 = (unsigned int)a.total_tiles;
+  } else {
+    a.sched.per_wave = (unsigned int)(a.total_tiles * 2 / 5 / n_waves);
+    a.sched.extra = 0;
+    a.sched.dyn0 = (unsigned int)(a.sched.per_wave * n_waves);
+    hipLaunchKernelGGL(reset_queue_kernel, dim3(1), dim3(64), 0, s, a.queue);
+  }
   hipLaunchKernelGGL(fn, dim3(groups), dim3(kWave * wpg), solve_lds_bytes(m, wpg), s, a);
   return hipGetLastError();
 }
