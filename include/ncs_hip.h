@@ -182,7 +182,8 @@ int ncs_hip_reduce_frames_device(ncs_ctx *ctx, const ncs_frame *frames,
 /* ncs_hip_reduce_frames_device without allocation.  No counterpart in the
  * reference: for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
- * work-queue counters and the frame table live in a fixed device array of
+ * work-queue counters and a frame table past 32 frames (up to that it travels
+ * with the launch) live in a fixed device array of
  * the library (21,504 bytes per GPU, held until the process ends), written
  * by kernels; at most 256 frames per call; the learned (conv-net) start,
  * which needs a start buffer, is refused.  Every call on one GPU shares that

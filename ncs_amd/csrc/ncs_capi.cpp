@@ -16,7 +16,7 @@
 namespace ncs {
 int solve_waves_per_cu(int m, bool general, bool pad, bool f16, int wpg);
 hipError_t launch_solve(int m, bool general, bool pad, bool f16, unsigned int waves, int wpg,
-                        hipStream_t s, SolveArgs a);
+                        hipStream_t s, SolveArgs a, const FrameDev *inline_frames);
 hipError_t launch_adu_to_photons(const uint16_t *adu, const float *offset, const float *gain,
                                  float *out, long long n, hipStream_t s);
 hipError_t launch_gamma_from_camera(const float *var, const float *gain, float *gamma,
@@ -31,8 +31,7 @@ hipError_t net_forward(const float *x, float *y, void *acts, const void *packs, 
 hipError_t net_backward(const float *x, const void *acts, const float *gout, float *gP,
                         const void *packs, long long n, int cus, hipStream_t s);
 int net_forward_grid(long long n, int cus);
-hipError_t net_warm(const FrameDev *frames, int n_frames, long long total, float *u0,
-                    const void *packs, const float *P, int grid, hipStream_t s);
+hipError_t net_warm(const NetWarmArgs &a, const FrameDev *inline_frames, int grid, hipStream_t s);
 hipError_t launch_eval(bool general, const float *data, const float *gamma, const float *u,
                        const float *tables, float alpha, int n, float *cost, float *grad,
                        hipStream_t s);
@@ -590,11 +589,16 @@ static void schedule_small_first_fixed(const FrameDev *fd, int n, long long tota
   }
 }
 
-// Frame descriptors go to the device through a pinned staging copy; a batch
-// identical to the previous one (the common streaming / benchmark case) is
-// not uploaded again.  The staging buffer is rewritten only after the event of
-// its last copy has completed.
-static int upload_frames(ncs_ctx *ctx, const std::vector<FrameDev> &fd, hipStream_t s) {
+// Device frame table of a launch in *table: null for up to kInlineFrames
+// frames, which go with the launch.  More go to the device through a pinned
+// staging copy; a batch identical to the previous one (the common streaming /
+// benchmark case) is not uploaded again.  The staging buffer is rewritten only
+// after the event of its last copy has completed.
+static int upload_frames(ncs_ctx *ctx, const std::vector<FrameDev> &fd, hipStream_t s,
+                         const FrameDev **table) {
+  *table = nullptr;
+  if (fd.size() <= (size_t)kInlineFrames) return NCS_OK;
+  *table = ctx->frames.as<FrameDev>();
   const size_t bytes = fd.size() * sizeof(FrameDev);
   if (ctx->frames_valid && ctx->last_frames.size() == fd.size() &&
       std::memcmp(ctx->last_frames.data(), fd.data(), bytes) == 0)
@@ -611,6 +615,7 @@ static int upload_frames(ncs_ctx *ctx, const std::vector<FrameDev> &fd, hipStrea
     ctx->frames_staging_cap = bytes;
   }
   HIPCHK(ctx->frames.ensure(bytes));
+  *table = ctx->frames.as<FrameDev>();
   std::memcpy(ctx->frames_staging, fd.data(), bytes);
   ctx->frames_valid = false;
   HIPCHK(hipMemcpyAsync(ctx->frames.p, ctx->frames_staging, bytes, hipMemcpyHostToDevice, s));
@@ -669,7 +674,7 @@ static Schedule resolve_schedule(const ncs_ctx *ctx, const ncs_params *p, bool p
 
 static SolveArgs make_args(const ncs_ctx *ctx, const FrameDev *d_frames, int n_frames,
                            long long total, const ncs_params *p, const float *u0,
-                           float *u_tiles, int *iters, int *status, float *cost,
+                           int *iters, int *status, float *cost,
                            unsigned int *queue) {
   SolveArgs a;
   a.frames = d_frames;
@@ -678,13 +683,12 @@ static SolveArgs make_args(const ncs_ctx *ctx, const FrameDev *d_frames, int n_f
   a.queue = queue;
   a.tables = ctx->tables.as<float>();
   a.u0 = u0;
-  a.u_tiles = u_tiles;
   a.iterations = iters;
   a.status = status;
   a.cost = cost;
-  a.evaluations = nullptr;
   a.max_it = p->max_iterations;
   a.eps = p->epsilon;
+  a.eps2 = p->epsilon * p->epsilon;
   a.ls = p->linesearch;
   a.max_ls = p->max_linesearch;
   a.ftol = p->ftol;
@@ -705,23 +709,26 @@ static SolveArgs make_args(const ncs_ctx *ctx, const FrameDev *d_frames, int n_f
 }
 
 static hipError_t launch_schedule(const ncs_ctx *ctx, const Schedule &sc, bool pad,
-                                  long long total, hipStream_t s, const SolveArgs &a) {
+                                  long long total, hipStream_t s, const SolveArgs &a,
+                                  const FrameDev *inline_frames = nullptr) {
   long long waves = (long long)sc.waves_per_cu * ctx->cus;
   waves = std::max<long long>(1, std::min(waves, total));
-  return launch_solve(sc.history, ctx->general, pad, sc.f16, (unsigned int)waves, sc.wpg, s, a);
+  return launch_solve(sc.history, ctx->general, pad, sc.f16, (unsigned int)waves, sc.wpg, s, a,
+                      inline_frames);
 }
 
-// Enqueue one persistent solve over device frames already described in
-// d_frames (device copy of fd).
-static int enqueue_solve(ncs_ctx *ctx, const FrameDev *d_frames, int n_frames, bool pad,
-                         long long total, const ncs_params *p, const float *u0,
-                         float *u_tiles, int *iters, int *status, float *cost,
+// Enqueue one persistent solve of the frames in d_frames (device table), or of
+// the n_frames <= kInlineFrames at inline_frames (host) when that is null.
+static int enqueue_solve(ncs_ctx *ctx, const FrameDev *d_frames, const FrameDev *inline_frames,
+                         int n_frames, bool pad, long long total, const ncs_params *p,
+                         const float *u0, int *iters, int *status, float *cost,
                          unsigned int *queue, hipStream_t s) {
   if (!ctx->has_mask) return fail(NCS_E_NOMASK, "no OTF mask set");
   if (total <= 0) return NCS_OK;
-  SolveArgs a = make_args(ctx, d_frames, n_frames, total, p, u0, u_tiles, iters, status, cost,
+  SolveArgs a = make_args(ctx, d_frames, n_frames, total, p, u0, iters, status, cost,
                           queue);
-  HIPCHK(launch_schedule(ctx, resolve_schedule(ctx, p, pad, total), pad, total, s, a));
+  HIPCHK(launch_schedule(ctx, resolve_schedule(ctx, p, pad, total), pad, total, s, a,
+                         inline_frames));
   return NCS_OK;
 }
 
@@ -752,19 +759,20 @@ extern "C" int ncs_hip_reduce_frames_device(ncs_ctx *ctx, const ncs_frame *frame
   hipStream_t s = (hipStream_t)stream;  // 0 = the default (NULL) stream
   HIPCHK(order_after_previous(ctx, s));
   schedule_small_first(fd, total);
-  rc = upload_frames(ctx, fd, s);
+  const FrameDev *table = nullptr;
+  rc = upload_frames(ctx, fd, s, &table);
   if (rc) return rc;
   const float *u0 = params->start == NCS_START_TILES ? u0_tiles : nullptr;
   if (params->start == NCS_START_LEARNED) {
     HIPCHK(ctx->u0_buf.ensure((size_t)total * kTilePix * sizeof(float)));
     const int grid = net_forward_grid(total, ctx->cus);
-    HIPCHK(net_warm(ctx->frames.as<FrameDev>(), n_frames, total, ctx->u0_buf.as<float>(),
-                    ctx->net_packs.p, ctx->net_params.as<float>(), grid, s));
+    HIPCHK(net_warm({table, n_frames, total, ctx->u0_buf.as<float>(), ctx->net_packs.p,
+                     ctx->net_params.as<float>()}, fd.data(), grid, s));
     u0 = ctx->u0_buf.as<float>();
   }
-  rc = enqueue_solve(ctx, ctx->frames.as<FrameDev>(), n_frames, any_pad(ctx, frames, n_frames),
-                     total, params, u0, nullptr,
-                     iterations, status, cost, ctx->queue.as<unsigned int>(), s);
+  rc = enqueue_solve(ctx, table, fd.data(), n_frames, any_pad(ctx, frames, n_frames), total,
+                     params, u0, iterations, status, cost,
+                     ctx->queue.as<unsigned int>(), s);
   if (rc) return rc;
   HIPCHK(mark_solve(ctx, s));
   return NCS_OK;
@@ -806,6 +814,8 @@ extern "C" int ncs_hip_reduce_frames_device_noalloc(ncs_ctx *ctx, const ncs_fram
   unsigned int *dq = static_cast<unsigned int *>(ctx->scratch);
   FrameDev *dfr =
       reinterpret_cast<FrameDev *>(static_cast<unsigned char *>(ctx->scratch) + kScratchFrameOffset);
+  const bool inl = n_frames <= kInlineFrames;
+  FrameDev sorted[kInlineFrames];
   long long first = 0;  // schedule position of the next frame's first tile
   for (int i0 = 0; i0 < n_frames; i0 += kFramesPerWrite) {
     FrameChunk c;
@@ -816,15 +826,17 @@ extern "C" int ncs_hip_reduce_frames_device_noalloc(ncs_ctx *ctx, const ncs_fram
       c.f[k] = fd[i];
       c.f[k].first = first;
       first += frame_tiles(fd, n_frames, total, i);
+      if (inl) sorted[i0 + k] = c.f[k];
     }
+    if (inl) continue;
     hipLaunchKernelGGL(write_frames_kernel, dim3(1), dim3(64), 0, s, c, dfr);
     HIPCHK(hipGetLastError());
   }
   // the counters, where the launch needs them, are reset by a kernel before
   // the solve (launch_solve)
-  return enqueue_solve(ctx, dfr, n_frames, any_pad(ctx, frames, n_frames), total, params,
-                       params->start == NCS_START_TILES ? u0_tiles : nullptr, nullptr,
-                       iterations, status, cost, dq, s);
+  return enqueue_solve(ctx, inl ? nullptr : dfr, sorted, n_frames,
+                       any_pad(ctx, frames, n_frames), total, params,
+                       params->start == NCS_START_TILES ? u0_tiles : nullptr, iterations, status, cost, dq, s);
 }
 
 extern "C" int ncs_hip_solve_tiles_device(ncs_ctx *ctx, const float *data_in,
@@ -917,10 +929,11 @@ extern "C" int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int 
     fd[i].ds = fd[i].gs = fd[i].os = f.width;
   }
   schedule_small_first(fd, total);
-  rc = upload_frames(ctx, fd, s);
+  const FrameDev *table = nullptr;
+  rc = upload_frames(ctx, fd, s, &table);
   if (rc) return rc;
-  rc = enqueue_solve(ctx, ctx->frames.as<FrameDev>(), n_frames, any_pad(ctx, frames, n_frames),
-                     total, params, nullptr, nullptr, ctx->iters.as<int>(), ctx->status.as<int>(),
+  rc = enqueue_solve(ctx, table, fd.data(), n_frames, any_pad(ctx, frames, n_frames), total,
+                     params, nullptr, ctx->iters.as<int>(), ctx->status.as<int>(),
                      ctx->cost.as<float>(), ctx->queue.as<unsigned int>(), s);
   if (rc) {
     (void)hipStreamSynchronize(s);
@@ -1038,11 +1051,12 @@ extern "C" int ncs_hip_net_predict_frames_device(ncs_ctx *ctx, const ncs_frame *
   HIPCHK(set_device(ctx));
   hipStream_t s = (hipStream_t)stream;
   schedule_small_first(fd, total);
-  rc = upload_frames(ctx, fd, s);
+  const FrameDev *table = nullptr;
+  rc = upload_frames(ctx, fd, s, &table);
   if (rc) return rc;
   const int grid = net_forward_grid(total, ctx->cus);
-  HIPCHK(net_warm(ctx->frames.as<FrameDev>(), n_frames, total, u0_tiles, ctx->net_packs.p,
-                  ctx->net_params.as<float>(), grid, s));
+  HIPCHK(net_warm({table, n_frames, total, u0_tiles, ctx->net_packs.p,
+                   ctx->net_params.as<float>()}, fd.data(), grid, s));
   return NCS_OK;
 }
 
@@ -1169,7 +1183,7 @@ extern "C" int ncs_hip_autotune(ncs_ctx *ctx, const ncs_frame *frames, int n_fra
     return fail(NCS_E_HIP, std::string("autotune setup: ") + hipGetErrorString(e));
   }
   const SolveArgs a = make_args(ctx, dfr.as<FrameDev>(), n_frames, total, base, nullptr,
-                                nullptr, nullptr, nullptr, nullptr, q.as<unsigned int>());
+                                nullptr, nullptr, nullptr, q.as<unsigned int>());
   // one untimed run (code load, caches), then the best of three
   auto time_one = [&](const Schedule &sc, float *ms) -> hipError_t {
     hipError_t r = launch_schedule(ctx, sc, pad, total, s, a);
@@ -1554,13 +1568,13 @@ static int capture_replay(ncs_pipeline *pl, hipGraph_t *out) {
   const float *u0 = nullptr;
   if (e == hipSuccess && pl->learned) {
     const int grid = net_forward_grid(pl->total, ctx->cus);
-    e = net_warm(pl->frames.as<FrameDev>(), pl->n, pl->total, pl->u0.as<float>(),
-                 ctx->net_packs.p, ctx->net_params.as<float>(), grid, s);
+    e = net_warm({pl->frames.as<FrameDev>(), pl->n, pl->total, pl->u0.as<float>(),
+                  ctx->net_packs.p, ctx->net_params.as<float>()}, nullptr, grid, s);
     u0 = pl->u0.as<float>();
   }
   if (e == hipSuccess) {
     const SolveArgs a = make_args(ctx, pl->frames.as<FrameDev>(), pl->n, pl->total, &pl->params,
-                                  u0, nullptr, pl->results.as<int>(),
+                                  u0, pl->results.as<int>(),
                                   pl->results.as<int>() + pl->total,
                                   pl->results.as<float>() + 2 * pl->total,
                                   pl->queue.as<unsigned int>());

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include "../../include/ncs_hip.h"
@@ -67,22 +68,31 @@ struct TileSchedule {
   unsigned int dyn0;
 };
 
+// Arguments of the conv net's kernel over frames.
+struct NetWarmArgs {
+  const FrameDev *frames;      // device table, or nullptr: the inline one
+  int n_frames;
+  long long total;
+  float *u0;                   // [tiles][256]
+  const void *packs;
+  const float *params;
+};
+
 // Solver parameters in the kernel's units.
 struct SolveArgs {
-  const FrameDev *frames;
+  const FrameDev *frames;      // device table, or nullptr: the inline one
   int n_frames;
   long long total_tiles;
   TileSchedule sched;          // filled in by launch_solve
   unsigned int *queue;         // kQueues work-queue counters (kQueueBytes)
   const float *tables;         // [64][16] per-lane OTF/DFT tables
   const float *u0;             // [tiles][256] warm start or nullptr
-  float *u_tiles;              // [tiles][256] solved tiles or nullptr
   int *iterations;             // [tiles] or nullptr
   int *status;                 // [tiles] or nullptr
   float *cost;                 // [tiles] or nullptr
-  int *evaluations;            // [tiles] or nullptr
   int max_it;
   float eps;
+  float eps2;                  // eps^2
   int ls;
   int max_ls;
   float ftol, gtol, xtol, min_step, max_step, stepm;
@@ -95,5 +105,41 @@ struct SolveArgs {
   int lin_slope;               // nonzero: the coefficients follow alpha
   float k_norm;                // bound on the NC Hessian's norm (row sums of the mask tables)
 };
+
+// A frame table of up to kInlineFrames frames travels in the kernel's
+// arguments (read by scalar loads from the kernel-argument segment): no copy
+// to the device before the launch and no table shared between launches.
+// Larger ones are in device memory (`frames`).
+constexpr int kInlineFrames = 32;
+
+template <class Args>
+struct WithFrames {
+  Args args;
+  FrameDev inl[kInlineFrames];
+};
+static_assert(sizeof(WithFrames<SolveArgs>) <= 4096, "kernel argument too large");
+
+// Fills the inline table from n frames in host memory.
+template <class Args>
+inline void set_inline(WithFrames<Args> &w, const FrameDev *frames, int n) {
+  for (int i = 0; i < n; i++) w.inl[i] = frames[i];
+}
+
+#if defined(__HIPCC__)
+// The frame table seen through the constant address space (scalar loads into
+// SGPRs; no kernel writes it).
+typedef __attribute__((address_space(4))) const FrameDev FrameConst;
+
+// The table of a kernel whose only argument is a WithFrames<Args>: `frames`,
+// or the inline one when that is null.
+template <class Args>
+__device__ __forceinline__ const FrameConst *frame_table(const FrameDev *frames) {
+  typedef __attribute__((address_space(4))) const char ConstByte;
+  const FrameConst *inl =
+      (const FrameConst *)((ConstByte *)__builtin_amdgcn_kernarg_segment_ptr() +
+                           offsetof(WithFrames<Args>, inl));
+  return frames != nullptr ? (const FrameConst *)frames : inl;
+}
+#endif
 
 }  // namespace ncs

@@ -426,35 +426,33 @@ void net_fwd_kernel(const float *__restrict__ xin, float *__restrict__ yout,
   }
 }
 
-typedef __attribute__((address_space(4))) const FrameDev FrameConstN;
-
 // Inference mode over frames: gather each window exactly like the solver,
 // normalise, run the net and write u0 = d + sigma * y as [tiles][256].
 __global__ __launch_bounds__(64 * kNetWaves) __attribute__((amdgpu_waves_per_eu(2)))
-void net_warm_kernel(const FrameDev *__restrict__ frames, int n_frames, long long total,
-                     float *__restrict__ u0, const i4 *__restrict__ packs,
-                     const float *__restrict__ P) {
+void net_warm_kernel(WithFrames<NetWarmArgs> W) {
+  const long long total = W.args.total;
+  float *__restrict__ u0 = W.args.u0;
+  const i4 *__restrict__ packs = reinterpret_cast<const i4 *>(W.args.packs);
+  const float *__restrict__ P = W.args.params;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   i4 *pk = reinterpret_cast<i4 *>(lds_raw);
   float *bl = reinterpret_cast<float *>(pk + kFwdPacks * 64);
   // the wave index is uniform: read it into a scalar register so the tile
   // loop's index arithmetic and frame-table reads stay on the scalar unit
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  // the frame table through the constant address space (scalar loads; the
-  // kernel never writes it)
-  const FrameConstN *fc = (const FrameConstN *)frames;
+  const FrameConst *fc = frame_table<NetWarmArgs>(W.args.frames);
   float *io = bl + 128 + wave * kNetWaveFloats;
   float *dkeep = io + kNetIoFloats;
   const int col = lane & 15, grp = lane >> 4;
   stage_forward(packs, P, pk, bl);
   for (long long t = (long long)blockIdx.x * kNetWaves + wave; t < total;
        t += (long long)gridDim.x * kNetWaves) {
-    int lo = 0, hi = n_frames - 1;
+    int lo = 0, hi = W.args.n_frames - 1;
     while (lo < hi) {
       int mid = (lo + hi + 1) >> 1;
       if (fc[mid].first <= t) lo = mid; else hi = mid - 1;
     }
-    const FrameConstN &F = fc[lo];
+    const FrameConst &F = fc[lo];
     const int local = (int)(t - F.first);  // a frame has fewer than 2^31 windows
     const int a = local / F.ty, b = local - a * F.ty;
     int bx, by, hv = 16, wv = 16;
@@ -959,12 +957,14 @@ hipError_t net_backward(const float *x, const void *acts, const float *gout, flo
   return hipGetLastError();
 }
 
-hipError_t net_warm(const FrameDev *frames, int n_frames, long long total, float *u0,
-                    const void *packs, const float *P, int grid, hipStream_t s) {
-  if (total <= 0) return hipSuccess;
-  hipLaunchKernelGGL(net_warm_kernel, dim3(grid), dim3(64 * kNetWaves), kNetFwdLdsBytes, s,
-                     frames, n_frames,
-                     total, u0, reinterpret_cast<const i4 *>(packs), P);
+// The starts of every tile of a.n_frames frames: at a.frames (device), or
+// without that at most kInlineFrames at inline_frames (host).
+hipError_t net_warm(const NetWarmArgs &a, const FrameDev *inline_frames, int grid, hipStream_t s) {
+  if (a.total <= 0) return hipSuccess;
+  WithFrames<NetWarmArgs> W;
+  W.args = a;
+  if (a.frames == nullptr) set_inline(W, inline_frames, a.n_frames);
+  hipLaunchKernelGGL(net_warm_kernel, dim3(grid), dim3(64 * kNetWaves), kNetFwdLdsBytes, s, W);
   return hipGetLastError();
 }
 

@@ -121,6 +121,7 @@ __device__ __forceinline__ float wave_dot(const float (&a)[4], const float (&b)[
 }
 
 __device__ __forceinline__ float rcpf(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ float sqrt_hw(float x) { return __builtin_amdgcn_sqrtf(x); }
 
 // Natural log of a normal, positive float on the transcendental unit:
 // v_log_f32 (log2) times ln 2, two instructions.  The libm-accurate logf
@@ -577,7 +578,8 @@ __device__ bool mt_cstep(float &stx, float &fx, float &dx, float &sty, float &fy
   return true;
 }
 
-__device__ __forceinline__ void mt_init(MtState &S, float dginit, const SolveArgs &A) {
+template <class AR>
+__device__ __forceinline__ void mt_init(MtState &S, float dginit, const AR &A) {
   S.stx = S.sty = 0.0f;
   S.fx = S.fy = 0.0f;
   S.dx = S.dy = dginit;
@@ -592,7 +594,8 @@ __device__ __forceinline__ void mt_init(MtState &S, float dginit, const SolveArg
 }
 
 // Clamp / fall back before a trial; returns the step to evaluate.
-__device__ __forceinline__ float mt_pre(MtState &S, float stp, const SolveArgs &A) {
+template <class AR>
+__device__ __forceinline__ float mt_pre(MtState &S, float stp, const AR &A) {
   if (S.brackt) {
     S.stmin = fminf(S.stx, S.sty);
     S.stmax = fmaxf(S.stx, S.sty);
@@ -611,8 +614,8 @@ __device__ __forceinline__ float mt_pre(MtState &S, float stp, const SolveArgs &
 
 // Tests after a trial (f = phi(stp), dg = phi'(stp)); on LS_CONTINUE the
 // next trial step is left in stp.
-__device__ __forceinline__ int mt_post(MtState &S, float &stp, float f, float dg,
-                                       const SolveArgs &A) {
+template <class AR>
+__device__ __forceinline__ int mt_post(MtState &S, float &stp, float f, float dg, const AR &A) {
   const float ftest1 = stp * S.dgtest;
   S.count++;
   if (S.brackt && ((stp <= S.stmin || S.stmax <= stp) || S.uinfo))
@@ -655,9 +658,6 @@ __device__ __forceinline__ int mt_post(MtState &S, float &stp, float f, float dg
 
 // Dynamic ranges a wave takes tiles from: its home range and the next one.
 constexpr int kScan = 2;
-
-// The frame table seen through the constant address space (scalar loads).
-typedef __attribute__((address_space(4))) const FrameDev FrameConst;
 
 struct TileGeom {
   int bx, by;           // window origin in the frame (may be -1)
@@ -809,7 +809,18 @@ __device__ __forceinline__ typename Basis32<F16>::type basis32(const LdsTables<F
 template <int M, bool GEN, bool PAD, bool F16>
 __global__ __launch_bounds__(64 * kMaxWavesPerGroup)
 __attribute__((amdgpu_waves_per_eu(M <= 4 ? 5 : 4, 8)))
-void solve_kernel(SolveArgs A) {
+void solve_kernel(WithFrames<SolveArgs> L) {
+  // The arguments are read from the kernel-argument segment where they are
+  // needed, through a pointer the compiler cannot see through: hoisted to the
+  // kernel's start they took 50 scalar registers more than there are, spilled
+  // to vector lanes and read back one VALU instruction at a time.
+  typedef __attribute__((address_space(4))) const SolveArgs ArgsConst;
+  auto args = []() -> ArgsConst & {
+    ArgsConst *a = (ArgsConst *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    return *a;
+  };
+  (void)L;
   extern __shared__ float4 lds_hist[];
   __shared__ MtState mt_state[kMaxWavesPerGroup];  // line-search state per wave
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform
@@ -825,15 +836,16 @@ void solve_kernel(SolveArgs A) {
   // OTF / DFT tables: each wave writes its lanes' entries (the same values
   // for every wave of the group) and each lane reads back only its own, so
   // no barrier is needed.
+  ArgsConst &A0 = args();
   typedef LdsTables<F16> TT;
   __shared__ f4 tab_lds[kWave * TT::kCount];
   {
-    const f4 *tb = reinterpret_cast<const f4 *>(A.tables + lane * 4 * kTableF4) + TT::kFirst;
+    const f4 *tb = reinterpret_cast<const f4 *>(A0.tables + lane * 4 * kTableF4) + TT::kFirst;
 #pragma unroll
     for (int i = 0; i < TT::kCount; i++) tab_lds[lane * TT::kCount + i] = tb[i];
   }
   const TT T{tab_lds + lane * TT::kCount};
-  const auto GB = basis32<F16>(T, A.tables);
+  const auto GB = basis32<F16>(T, A0.tables);
 
   // next_tile() gives the wave's next tile (uniform) or -1 when its static
   // block [next, end) and the dynamic ranges it takes from are exhausted
@@ -845,12 +857,13 @@ void solve_kernel(SolveArgs A) {
   unsigned int next, end;
   {
     const unsigned int w = blockIdx.x * (blockDim.x >> 6) + wave;
-    next = w * A.sched.per_wave + min(w, A.sched.extra);
-    end = next + A.sched.per_wave + (w < A.sched.extra ? 1u : 0u);
+    next = w * A0.sched.per_wave + min(w, A0.sched.extra);
+    end = next + A0.sched.per_wave + (w < A0.sched.extra ? 1u : 0u);
   }
   int qv = 0;  // dynamic ranges found exhausted
   auto next_tile = [&]() -> long long {
     if (next < end) return (long long)(next++);
+    ArgsConst &A = args();
     const unsigned int dyn0 = A.sched.dyn0, nd = (unsigned int)A.total_tiles - dyn0;
     if (nd == 0) return -1;
     for (; qv < kScan; qv++) {
@@ -865,14 +878,14 @@ void solve_kernel(SolveArgs A) {
     return -1;
   };
 
-  // The frame table is read through the constant address space (scalar
-  // loads into SGPRs; the kernel never writes it).  Tiles of a chunk are
-  // consecutive, so the previous frame is tried before a binary search.
-  const FrameConst *frames = (const FrameConst *)(A.frames);
+  // A wave's static tiles are consecutive, so the previous frame is tried
+  // before a binary search.
+  const FrameConst *frames = frame_table<SolveArgs>(A0.frames);
   int fi = 0;
   auto frame_of = [&](long long t) -> int {
-    if (!(frames[fi].first <= t && (fi + 1 >= A.n_frames || frames[fi + 1].first > t))) {
-      int lo = 0, hi = A.n_frames - 1;
+    const int n_frames = args().n_frames;
+    if (!(frames[fi].first <= t && (fi + 1 >= n_frames || frames[fi + 1].first > t))) {
+      int lo = 0, hi = n_frames - 1;
       while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
         if (frames[mid].first <= t) lo = mid; else hi = mid - 1;
@@ -916,8 +929,9 @@ void solve_kernel(SolveArgs A) {
         gg[r] = ok ? F.gamma[gr * (unsigned int)F.gs + gc] : 0.0f;
       }
     }
-    if (A.u0 != nullptr) {
-      const float *w = A.u0 + (F.slot + (t - F.first)) * kTilePix;  // uniform
+    const float *u0 = args().u0;
+    if (u0 != nullptr) {
+      const float *w = u0 + (F.slot + (t - F.first)) * kTilePix;  // uniform
 #pragma unroll
       for (int r = 0; r < 4; r++) w0[r] = w[(unsigned int)((4 * grp + r) * kTile + col)];
     }
@@ -931,6 +945,7 @@ void solve_kernel(SolveArgs A) {
   load_tile(frames[fc], G, t, raw_d, gm, w0);
 
   for (;;) {
+    ArgsConst &A = args();
     const FrameConst &F = frames[fc];
     const float alpha = F.alpha;
     float c[4], lin[4], u[4];
@@ -1042,7 +1057,7 @@ void solve_kernel(SolveArgs A) {
       for (int r = 0; r < 4; r++) gs[r] = fmaf(alpha, gncs[r], gls[r]);
     }
 
-    int status = NCS_REACHED_MAXITERS, iters = 0, evals = 1;
+    int status = NCS_REACHED_MAXITERS, iters = 0;
     bool gnc_exact = true;
     int n_inc = 0;  // incremental NC-gradient updates since the last exact one
     float gg, uu, kappa;
@@ -1055,7 +1070,7 @@ void solve_kernel(SolveArgs A) {
       uu = red[1];
       kappa = red[2] * (1.0f / 256.0f);
     }
-    bool done = gg <= A.eps * A.eps * fmaxf(1.0f, uu);
+    bool done = gg <= A.eps2 * fmaxf(1.0f, uu);
     float uu_max = uu;  // largest |u|^2 of the iterates
     if (done) status = NCS_SUCCESS;
     else if (gg <= kF16Floor * kF16Floor * fmaxf(1.0f, uu)) exact = true;
@@ -1065,7 +1080,7 @@ void solve_kernel(SolveArgs A) {
     float ds[4];  // search direction, spectral
 #pragma unroll
     for (int r = 0; r < 4; r++) ds[r] = -gs[r];
-    float step = rsqrtf(gg);
+    float step = 1.0f;
     // The spectral H0 (precond) models the likelihood curvature by its tile
     // mean.  From a start far from the solution that mean can change by
     // orders of magnitude along the way and the line search then fail; a
@@ -1080,7 +1095,8 @@ void solve_kernel(SolveArgs A) {
         h0_corr<GEN, true>(ds, T, GB, c, iv, u, gm, kappa, alpha, st, exact, Hz);
       else
         h0_spec<GEN>(ds, T, kappa, alpha);
-      step = 1.0f;
+    } else {
+      step = rsqrtf(gg);
     }
     float ys_last = 1.0f, yy_last = 1.0f;
 
@@ -1104,7 +1120,12 @@ void solve_kernel(SolveArgs A) {
         if (dg0 <= 0.0f || attempt == 1 || nh == 0) break;
         nh = 0;
 #pragma unroll
-        for (int r = 0; r < 4; r++) ds[r] = -gs[r];
+        for (int r = 0; r < 4; r++) {
+          ds[r] = -gs[r];
+          // (rare: keeps the compiler from computing this direction, with its
+          // four reciprocals, ahead of every search)
+          asm volatile("" : "+v"(ds[r]));
+        }
         if (spec_h0) {
           h0_spec<GEN>(ds, T, kappa, alpha);
         } else {
@@ -1128,7 +1149,6 @@ void solve_kernel(SolveArgs A) {
       {
         float red[2];
         ll_trial<PAD, kCacheIv>(tstep, u, dp, gm, c, lin, iv, gt, ivt, red);
-        evals++;
         phi = red[0] + alpha * tstep * (a1 + 0.5f * tstep * a2);
         const float dphi = red[1] + alpha * (a1 + tstep * a2);
         if (A.ls == NCS_LS_MORE_THUENTE) {
@@ -1142,6 +1162,7 @@ void solve_kernel(SolveArgs A) {
             // LDS and the memory clobbers stop the compiler from holding it
             // in VGPRs across the vector trials.
             MtState &S_ = mt_lds;
+            ArgsConst &A = args();
             mt_init(S_, dg0, A);
             S_.stmin = 0.0f;
             S_.stmax = 5.0f * tstep;
@@ -1152,8 +1173,7 @@ void solve_kernel(SolveArgs A) {
               asm volatile("" ::: "memory");
               ll_trial<PAD, kCacheIv>(tstep, u, dp, gm, c, lin, iv, gt, ivt, red);
               asm volatile("" ::: "memory");
-              evals++;
-              phi = red[0] + alpha * tstep * (a1 + 0.5f * tstep * a2);
+                    phi = red[0] + alpha * tstep * (a1 + 0.5f * tstep * a2);
               const float dpt = red[1] + alpha * (a1 + tstep * a2);
               ls = mt_post(S_, tstep, phi, dpt, A);
               dphi_acc = dpt;
@@ -1161,6 +1181,7 @@ void solve_kernel(SolveArgs A) {
           }
         } else {
           // Armijo backtracking (ncs.cl:979-1035)
+          ArgsConst &A = args();
           int trials = 1;
           for (;;) {
             if (phi <= A.ftol * dg0 * tstep) {
@@ -1172,8 +1193,7 @@ void solve_kernel(SolveArgs A) {
             if (!(tstep >= A.min_step)) { ls = LS_FAIL_MINSTEP; break; }
             if (trials >= A.max_ls) { ls = LS_FAIL_PRECISION; break; }
             ll_trial<PAD, kCacheIv>(tstep, u, dp, gm, c, lin, iv, gt, ivt, red);
-            evals++;
-            trials++;
+                trials++;
             phi = red[0] + alpha * tstep * (a1 + 0.5f * tstep * a2);
           }
         }
@@ -1220,7 +1240,7 @@ void solve_kernel(SolveArgs A) {
         kappa = red[2] * (1.0f / 256.0f);
         gnc_exact = true;
         n_inc = 0;
-        if (gg <= A.eps * A.eps * fmaxf(1.0f, uu)) {
+        if (gg <= A.eps2 * fmaxf(1.0f, uu)) {
           // the exact gradient already meets the stop rule at u (the point
           // the previous iteration accepted, or the plain start)
           iters = k - 1;
@@ -1258,8 +1278,6 @@ void solve_kernel(SolveArgs A) {
         ut[r] = u[r] + tstep * dp[r];
         gncn[r] = fmaf(tstep, gncn[r], gncs[r]);
       }
-      const bool moved = __any((ut[0] != u[0]) | (ut[1] != u[1]) | (ut[2] != u[2]) |
-                               (ut[3] != u[3]));
       gnc_exact = false;
       n_inc++;
       if ((k & 15) == 0) {  // periodic exact refresh of the NC gradient
@@ -1292,7 +1310,7 @@ void solve_kernel(SolveArgs A) {
         uu_max = fmaxf(uu_max, uu);
         kappa = red[2] * (1.0f / 256.0f);
         yy = red[2];
-        done = gg <= A.eps * A.eps * fmaxf(1.0f, uu);
+        done = gg <= A.eps2 * fmaxf(1.0f, uu);
         if (!done && gg <= kF16Floor * kF16Floor * fmaxf(1.0f, uu)) exact = true;
         if (!done || gnc_exact) break;
         // The incremental NC gradient differs from K u by rounding, at most
@@ -1301,8 +1319,10 @@ void solve_kernel(SolveArgs A) {
         // bound, an exact NC gradient would confirm convergence too;
         // otherwise confirm with one.  (The FP16 build always confirms: the
         // bound's registers cost it more spills than the refresh.)
-        if (!F16 && sqrtf(gg) + (float)n_inc * kNcDrift * alpha * A.k_norm * sqrtf(uu_max) <=
-                        A.eps * fmaxf(1.0f, sqrtf(uu)))
+        // The square roots are the hardware's (1 ulp, one instruction where
+        // the exact one takes fifteen): the bound has a factor of 2 to spare.
+        if (!F16 && sqrt_hw(gg) + (float)n_inc * kNcDrift * alpha * A.k_norm * sqrt_hw(uu_max) <=
+                        A.eps * fmaxf(1.0f, sqrt_hw(uu)))
           break;
         to_spec16<false>(ut, T, GB, st, zs, exact);
         nc_spec<GEN>(zs, T, gncn);
@@ -1310,6 +1330,8 @@ void solve_kernel(SolveArgs A) {
         n_inc = 0;
       }
       // history pair: s = t d, y = g_new - g (spectral)
+      const bool moved = done || __any((ut[0] != u[0]) | (ut[1] != u[1]) | (ut[2] != u[2]) |
+                                       (ut[3] != u[3]));
       const bool added = ys > 0.0f && !done && moved && k != A.max_it;
       if (added) {
         head = (head + 1 == M) ? 0 : head + 1;
@@ -1413,20 +1435,17 @@ void solve_kernel(SolveArgs A) {
     asm volatile("" : "+v"(ln));
     const int col = ln & 15, grp = ln >> 4;
     const long long ts = F.slot + (t - F.first);
-    float *const ut_base = A.u_tiles != nullptr ? A.u_tiles + ts * kTilePix : nullptr;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int row = 4 * grp + r;
       if (F.out != nullptr && row >= G.r_lo && row < G.r_hi && col >= G.c_lo &&
           col < G.c_hi)
         F.out[(unsigned int)(G.bx + row) * (unsigned int)F.os + (unsigned int)(G.by + col)] = u[r];
-      if (ut_base != nullptr) ut_base[(unsigned int)(row * kTile + col)] = u[r];
     }
     if (lane == 0) {
       if (A.iterations) A.iterations[ts] = iters;
       if (A.status) A.status[ts] = status;
       if (A.cost) A.cost[ts] = f;
-      if (A.evaluations) A.evaluations[ts] = evals;
     }
     if (tn < 0) break;
     t = tn;
@@ -1505,7 +1524,7 @@ __global__ void reset_queue_kernel(unsigned int *q) {
 
 // Instantiations: history 1..8, with and without the odd-mask coupling and
 // zero-padded pixels, FP32 or FP16-split basis changes.
-typedef void (*SolveKernelFn)(SolveArgs);
+typedef void (*SolveKernelFn)(WithFrames<SolveArgs>);
 
 template <int M, bool F16>
 static SolveKernelFn pick2(bool general, bool pad) {
@@ -1550,7 +1569,8 @@ int solve_waves_per_cu(int m, bool general, bool pad, bool f16, int wpg) {
 }
 
 // Launches `waves` persistent waves in workgroups of `wpg` waves (waves is
-// rounded up to a multiple of wpg).
+// rounded up to a multiple of wpg).  Without a device frame table (a.frames
+// null) the a.n_frames <= kInlineFrames frames are at inline_frames (host).
 //
 // Shares of the tiles.  A device-scope atomic is resolved beyond the XCD's
 // L2, so tiles are assigned statically where that balances: up to
@@ -1565,7 +1585,7 @@ int solve_waves_per_cu(int m, bool general, bool pad, bool f16, int wpg) {
 // 120 and 87 us, 150 and 128 us.  Chunks of two or three were within 1% with
 // the linear start's short tiles and 2% slower with the plain start's.
 hipError_t launch_solve(int m, bool general, bool pad, bool f16, unsigned int waves, int wpg,
-                        hipStream_t s, SolveArgs a) {
+                        hipStream_t s, SolveArgs a, const FrameDev *inline_frames) {
   SolveKernelFn fn = solve_kernel_for(m, general, pad, f16);
   if (!fn || wpg < 1 || wpg > kMaxWavesPerGroup || waves == 0) return hipErrorInvalidValue;
   const unsigned int groups = (waves + wpg - 1) / wpg;
@@ -1581,7 +1601,10 @@ hipError_t launch_solve(int m, bool general, bool pad, bool f16, unsigned int wa
     a.sched.dyn0 = (unsigned int)(a.sched.per_wave * n_waves);
     hipLaunchKernelGGL(reset_queue_kernel, dim3(1), dim3(64), 0, s, a.queue);
   }
-  hipLaunchKernelGGL(fn, dim3(groups), dim3(kWave * wpg), solve_lds_bytes(m, wpg), s, a);
+  WithFrames<SolveArgs> L;
+  L.args = a;
+  if (a.frames == nullptr) set_inline(L, inline_frames, a.n_frames);
+  hipLaunchKernelGGL(fn, dim3(groups), dim3(kWave * wpg), solve_lds_bytes(m, wpg), s, L);
   return hipGetLastError();
 }
 
