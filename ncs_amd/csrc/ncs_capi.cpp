@@ -527,6 +527,7 @@ static int describe_frames(const ncs_ctx *ctx, const ncs_frame *frames, int n, F
     d.alpha = f.alpha;
     d.geom = f.geometry;
     d.ty = (int)tiles_axis(f.width, f.geometry, win);
+    d.ty_magic = div_magic((unsigned int)d.ty);
     d.win = win;
     d.first = total;
     d.slot = total;
@@ -1384,6 +1385,7 @@ extern "C" int ncs_hip_pipeline_create(ncs_ctx *ctx, const ncs_pipeline_frame *f
     d.alpha = f.alpha;
     d.geom = f.geometry;
     d.ty = (int)tiles_axis(f.width, f.geometry, ctx->win);
+    d.ty_magic = div_magic((unsigned int)d.ty);
     d.win = ctx->win;
     d.first = pl->total;
     d.slot = pl->total;

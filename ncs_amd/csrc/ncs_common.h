@@ -38,6 +38,26 @@ constexpr int kTableSlope = 10;
 constexpr int kTableLaneFloats = 4 * kTableF4;
 constexpr int kTableFloats = kWave * kTableLaneFloats;
 
+// Division of n < 2^31 by d >= 1 with one multiplication (Granlund and
+// Montgomery 1994): with l = ceil(log2 d) and m = floor(2^(31 + l) / d) + 1,
+// n / d = (n m) >> (31 + l).  d = 1 has no such m in 32 bits and takes 0.
+inline unsigned int div_magic(unsigned int d) {
+  if (d <= 1) return 0;
+  int l = 0;
+  while ((1ull << l) < d) l++;
+  // 2^(31 + l) / d by parts: l <= 31, the quotient is below 2^32
+  const unsigned long long p = 1ull << (31 + l);
+  return (unsigned int)(p / d + 1);
+}
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline unsigned int div_by(unsigned int n, unsigned int d, unsigned int magic) {
+  if (magic == 0) return n;
+  const unsigned int hi = (unsigned int)(((unsigned long long)n * magic) >> 32);
+  return hi >> (31 - __builtin_clz(d - 1));  // l - 1
+}
+
 // One frame of a batch, as the kernel sees it.  A batch's tiles are claimed
 // in frame-table order (`first`, increasing along the table); per-tile arrays
 // (warm starts, tile outputs, iterations, status, cost) are indexed in the
@@ -54,6 +74,7 @@ struct FrameDev {
   int ty;              // tiles along the fast axis
   int win;             // window side r of the reference geometry (even, 4..16);
                        // a window fills the top-left r x r of the 16 x 16 tile
+  unsigned int ty_magic;  // div_magic(ty)
   long long first;     // schedule position of the frame's first tile
   long long slot;      // per-tile array index of the frame's first tile
 };

@@ -454,7 +454,8 @@ void net_warm_kernel(WithFrames<NetWarmArgs> W) {
     }
     const FrameConst &F = fc[lo];
     const int local = (int)(t - F.first);  // a frame has fewer than 2^31 windows
-    const int a = local / F.ty, b = local - a * F.ty;
+    const int a = (int)div_by((unsigned int)local, (unsigned int)F.ty, F.ty_magic);
+    const int b = local - a * F.ty;
     int bx, by, hv = 16, wv = 16;
     if (F.geom == NCS_GEOM_REFERENCE) {
       bx = min(-1 + 14 * a, F.H - 15);

@@ -114,8 +114,14 @@ __device__ __forceinline__ float tile_scale(const float (&x)[4]) {
   return (e >= 5 && e <= 254) ? __uint_as_float((unsigned int)(259 - e) << 23) : 1.0f;
 }
 
+// The fused multiply-adds are written out: left to the compiler, which
+// product is fused changes with the surrounding code, and with it the last
+// bits of the iterates.  ODD fuses products 1 and 3 into 0 and 2, else the
+// other way round.
+template <bool ODD = false>
 __device__ __forceinline__ float wave_dot(const float (&a)[4], const float (&b)[4]) {
-  float s[1] = {a[0] * b[0] + a[1] * b[1] + (a[2] * b[2] + a[3] * b[3])};
+  float s[1] = {ODD ? fmaf(a[1], b[1], a[0] * b[0]) + fmaf(a[3], b[3], a[2] * b[2])
+                    : fmaf(a[0], b[0], a[1] * b[1]) + fmaf(a[2], b[2], a[3] * b[3])};
   wave_sum<1>(s);
   return s[0];
 }
@@ -447,11 +453,23 @@ __device__ __forceinline__ void h0_corr(float (&x)[4], const TT &T, const GB &G,
                                         const float (&c)[4], const float (&iv)[4],
                                         const float (&u)[4], const float (&gm)[4], float kappa,
                                         float alpha, float s, bool exact, float4 *stash) {
-  h0_spec<GEN>(x, T, kappa, alpha);
   float xp[4], w[4];
-  // P x waits in LDS across the two basis changes (registers are the
-  // scarcer resource there); the clobbers keep the compiler from
-  // forwarding the stored value instead of reloading it
+  // P x, and without partner coupling P itself, wait in LDS across the two
+  // basis changes (registers are the scarcer resource there); the clobbers
+  // keep the compiler from forwarding the stored values instead of reloading
+  // them
+  if constexpr (GEN) {
+    h0_spec<GEN>(x, T, kappa, alpha);
+  } else {
+    const f4 q = T.qe();
+    float pr[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      pr[r] = rcpf(fmaf(alpha, q[r], kappa));
+      x[r] *= pr[r];
+    }
+    stash[kWave] = make_float4(pr[0], pr[1], pr[2], pr[3]);
+  }
   *stash = make_float4(x[0], x[1], x[2], x[3]);
   asm volatile("" ::: "memory");
   to_pix16(x, T, G, s, xp, exact);
@@ -462,8 +480,16 @@ __device__ __forceinline__ void h0_corr(float (&x)[4], const TT &T, const GB &G,
     xp[r] *= fminf(c[r] * v * v, hi) - kappa;
   }
   to_spec16(xp, T, G, 1.0f, w, exact);
-  h0_spec<GEN>(w, T, kappa, alpha);
   asm volatile("" ::: "memory");
+  if constexpr (GEN) {
+    h0_spec<GEN>(w, T, kappa, alpha);
+  } else {
+    const float4 pr = stash[kWave];
+    w[0] *= pr.x;
+    w[1] *= pr.y;
+    w[2] *= pr.z;
+    w[3] *= pr.w;
+  }
   const float4 z = *stash;
   x[0] = z.x - w[0];
   x[1] = z.y - w[1];
@@ -665,11 +691,24 @@ struct TileGeom {
   int c_lo, c_hi;       // owned local cols
 };
 
+// Byte offset of tile row 4 grp for a row stride below 2^24 elements
+// (kRowStride24): one 24-bit multiply; below 2^32 bytes.
+constexpr int kRowStride24 = 1 << 24;
+__device__ __forceinline__ unsigned int row_bytes24(int grp, int stride) {
+  return __umul24((unsigned int)grp, (unsigned int)stride) * 16u;
+}
+// The element at a 32-bit byte offset from a uniform pointer.
+__device__ __forceinline__ const float &at_byte(const float *p, unsigned int off) {
+  return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(p) + off);
+}
+
 __device__ __forceinline__ TileGeom tile_geom(const FrameConst &F, long long local) {
   TileGeom G;
-  // tile indices fit 32 bits (the host caps a batch below 2^32 tiles)
+  // a frame has fewer than 2^31 windows; the division by ty is a
+  // multiplication by the host's reciprocal (div_magic): three scalar
+  // instructions instead of a VALU reciprocal sequence
   const unsigned int l32 = (unsigned int)local, ty = (unsigned int)F.ty;
-  const int a = (int)(l32 / ty), b = (int)(l32 - (unsigned int)a * ty);
+  const int a = (int)div_by(l32, ty, F.ty_magic), b = (int)(l32 - (unsigned int)a * ty);
   if (F.geom == NCS_GEOM_REFERENCE) {
     // windows of side r at -1, -1 + (r - 2), ...; the last one clamped to
     // end one pixel past the frame (ncs.c:71-85); each owns its interior up
@@ -753,18 +792,34 @@ __device__ __forceinline__ void ll_trial(float t, const float (&u)[4], const flo
                                          float (&gt)[4], float (&ivt)[4], float (&red)[2]) {
   red[0] = 0.0f;
   red[1] = 0.0f;
+  // v = max(u + gamma, FITMIN) before and at the step; without a pixel at
+  // the guard (nearly always) the maxima change nothing and delta is the exact
+  // step t d: one uniform branch instead of sixteen VALU per trial
+  float td[4], v0[4], vt[4], delta[4];
+  bool free[4];
 #pragma unroll
   for (int r = 0; r < 4; r++) {
-    const float td = t * dv[r];
-    const float w0 = u[r] + gm[r];
-    const float w = w0 + td;
-    const float vt = fmaxf(w, kFitMin);
-    // relative change of max(u + gamma, FITMIN); exact step t d when no guard
-    const float delta = (w0 >= kFitMin && w >= kFitMin) ? td : vt - fmaxf(w0, kFitMin);
-    const float lg = log1p_acc(delta * (CACHED ? iv[r] : rcpf(fmaxf(w0, kFitMin))));
+    td[r] = t * dv[r];
+    v0[r] = u[r] + gm[r];
+    vt[r] = v0[r] + td[r];
+    delta[r] = td[r];
+    free[r] = v0[r] >= kFitMin && vt[r] >= kFitMin;
+  }
+  if (!__all(free[0] && free[1] && free[2] && free[3])) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      asm volatile("" : "+v"(vt[r]));  // not ahead of the branch
+      vt[r] = fmaxf(vt[r], kFitMin);
+      v0[r] = fmaxf(v0[r], kFitMin);
+      if (!free[r]) delta[r] = vt[r] - v0[r];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const float lg = log1p_acc(delta[r] * (CACHED ? iv[r] : rcpf(v0[r])));
     const float l = PAD ? lin[r] : 1.0f;
-    red[0] += l * td - c[r] * lg;
-    ivt[r] = rcpf(vt);
+    red[0] += l * td[r] - c[r] * lg;
+    ivt[r] = rcpf(vt[r]);
     gt[r] = l - c[r] * ivt[r];
     red[1] += gt[r] * dv[r];
   }
@@ -776,23 +831,33 @@ __device__ __forceinline__ void ll_trial(float t, const float (&u)[4], const flo
 // (measured at history 5), and precond 2 runs as precond 1.
 constexpr int kCorrHistory = 3;
 
+// Histories from kRegPair on keep the newest pair in registers, which they
+// have to spare (109 of 128 at 5): the LDS of the other four pairs lets 16
+// waves share a CU instead of 12 (history 5, plain start, ten 2048^2 frames:
+// 1015 -> 907 us).
+constexpr int kRegPair = 5;
+__host__ __device__ constexpr int ring_slots(int m) { return m >= kRegPair ? m - 1 : m; }
+
 // LDS of one wave, in float4 per lane: the s and y vectors of the history,
-// and the stash of the curvature-corrected H0 where there is one.
+// and the stash of the curvature-corrected H0 (P x and P) where there is one.
 __host__ __device__ constexpr int wave_lds_f4(int m) {
-  return 2 * m + (m <= kCorrHistory ? 1 : 0);
+  return 2 * ring_slots(m) + (m <= kCorrHistory ? 2 : 0);
 }
 
 // One to kMaxWavesPerGroup waves per workgroup, each solving its own tiles;
 // a wave's L-BFGS history lives in its slice of LDS as two rings of M vectors,
-// followed by one vector of scratch for the curvature-corrected H0 (each
+// followed by the scratch of the curvature-corrected H0 (each
 // lane keeps its own 4 values at float4 index slot * 64 + lane, so no lane
 // reads another lane's LDS and no barrier is needed).  PAD enables
 // zero-padded pixels (block geometry).
 //
-// Occupancy target: 5 waves per SIMD (at most 96 VGPRs) for histories up to
-// 4, 4 waves (128 VGPRs) above; the latency of the reduction chains and of
-// the MFMA stages is hidden by other waves, so the extra wave pays
-// (measured: -10 % at history 1).
+// Occupancy target: 5 waves per SIMD (at most 96 VGPRs) at histories 1 and 2,
+// 4 waves (128 VGPRs) above: the latency of the reduction chains and of the
+// MFMA stages is hidden by other waves.  Linear start, ten 2048^2 frames,
+// history 1: 593 us with 5 waves (7 registers spilled), 615 with 4.  From
+// history 3 on the LDS of the histories allows 16 waves per CU and no more,
+// so the registers of a fifth would be lost to spills (history 3, plain
+// start: 902 us with 128 VGPRs, 926 with 96).
 //
 // F16 selects the basis changes: FP16 hi/lo split on the FP16 matrix cores
 // (FP32 near the stop rule and as fallback), or FP32 MFMA throughout.
@@ -808,7 +873,7 @@ __device__ __forceinline__ typename Basis32<F16>::type basis32(const LdsTables<F
 
 template <int M, bool GEN, bool PAD, bool F16>
 __global__ __launch_bounds__(64 * kMaxWavesPerGroup)
-__attribute__((amdgpu_waves_per_eu(M <= 4 ? 5 : 4, 8)))
+__attribute__((amdgpu_waves_per_eu(M <= 2 ? 5 : 4, 8)))
 void solve_kernel(WithFrames<SolveArgs> L) {
   // The arguments are read from the kernel-argument segment where they are
   // needed, through a pointer the compiler cannot see through: hoisted to the
@@ -827,9 +892,11 @@ void solve_kernel(WithFrames<SolveArgs> L) {
   constexpr bool kCacheIv = M <= 3;  // keep 1/(u+gamma) across iterations
   constexpr bool kCorr = M <= kCorrHistory;
   MtState &mt_lds = mt_state[wave];
-  float4 *const Sb = lds_hist + wave * (wave_lds_f4(M) * 64);  // s vectors, ring of M
-  float4 *const Yb = Sb + M * 64;                           // y vectors, ring of M
-  float4 *const Hz = Yb + M * 64 + (threadIdx.x & 63);      // this lane's H0 stash
+  constexpr bool kReg = M >= kRegPair;
+  constexpr int kRing = ring_slots(M);
+  float4 *const Sb = lds_hist + wave * (wave_lds_f4(M) * 64);  // s vectors, ring
+  float4 *const Yb = Sb + kRing * 64;                          // y vectors, ring
+  float4 *const Hz = Yb + kRing * 64 + (threadIdx.x & 63);     // this lane's H0 stash
   const int lane = threadIdx.x & 63;
   const int col = lane & 15, grp = lane >> 4;
 
@@ -904,6 +971,21 @@ void solve_kernel(WithFrames<SolveArgs> L) {
     int ln = lane;
     asm volatile("" : "+v"(ln));
     const int col = ln & 15, grp = ln >> 4;
+    // A whole window inside the frame (97% of a 2048^2 frame's): one lane
+    // offset in bytes from a scalar pointer per row.  The clamped form below
+    // takes two 64-bit multiply-adds per element, 45 VALU a tile more.
+    if (!PAD && G.bx >= 0 && G.by >= 0 && G.bx + kTile <= F.H && G.by + kTile <= F.W &&
+        (F.ds | F.gs) < kRowStride24) {
+      const float *const pd = F.data + ((long long)G.bx * F.ds + G.by);
+      const float *const pg = F.gamma + ((long long)G.bx * F.gs + G.by);
+      const unsigned int od = row_bytes24(grp, F.ds) + 4u * (unsigned int)col;
+      const unsigned int og = row_bytes24(grp, F.gs) + 4u * (unsigned int)col;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        dd[r] = at_byte(pd + (long long)r * F.ds, od);
+        gg[r] = at_byte(pg + (long long)r * F.gs, og);
+      }
+    } else
     // 32-bit element offsets from uniform base pointers (the host keeps
     // every frame below 2^31 elements)
 #pragma unroll
@@ -1076,7 +1158,8 @@ void solve_kernel(WithFrames<SolveArgs> L) {
     else if (gg <= kF16Floor * kF16Floor * fmaxf(1.0f, uu)) exact = true;
 
     float rho[M], al[M];  // rho[j], al[j]: j-th newest pair
-    int nh = 0, head = M - 1;
+    int nh = 0, head = kRing - 1;
+    float s0[4], y0[4];  // the newest pair (kReg)
     float ds[4];  // search direction, spectral
 #pragma unroll
     for (int r = 0; r < 4; r++) ds[r] = -gs[r];
@@ -1334,11 +1417,23 @@ void solve_kernel(WithFrames<SolveArgs> L) {
                                        (ut[3] != u[3]));
       const bool added = ys > 0.0f && !done && moved && k != A.max_it;
       if (added) {
-        head = (head + 1 == M) ? 0 : head + 1;
-        Sb[head * 64 + lane] = make_float4(tstep * ds[0], tstep * ds[1], tstep * ds[2],
-                                           tstep * ds[3]);
-        Yb[head * 64 + lane] = make_float4(gnews[0] - gs[0], gnews[1] - gs[1],
-                                           gnews[2] - gs[2], gnews[3] - gs[3]);
+        if (!kReg || nh > 0) head = (head + 1 == kRing) ? 0 : head + 1;
+        if constexpr (kReg) {
+          if (nh > 0) {
+            Sb[head * 64 + lane] = make_float4(s0[0], s0[1], s0[2], s0[3]);
+            Yb[head * 64 + lane] = make_float4(y0[0], y0[1], y0[2], y0[3]);
+          }
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            s0[r] = tstep * ds[r];
+            y0[r] = gnews[r] - gs[r];
+          }
+        } else {
+          Sb[head * 64 + lane] = make_float4(tstep * ds[0], tstep * ds[1], tstep * ds[2],
+                                             tstep * ds[3]);
+          Yb[head * 64 + lane] = make_float4(gnews[0] - gs[0], gnews[1] - gs[1],
+                                             gnews[2] - gs[2], gnews[3] - gs[3]);
+        }
       }
 #pragma unroll
       for (int r = 0; r < 4; r++) {
@@ -1360,22 +1455,37 @@ void solve_kernel(WithFrames<SolveArgs> L) {
         nh = min(nh + 1, M);
       }
 
+      // the j-th newest pair
+      auto pair = [&](int j, float (&sj)[4], float (&yj)[4]) {
+        if (kReg && j == 0) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            sj[r] = s0[r];
+            yj[r] = y0[r];
+          }
+          return;
+        }
+        const int back = kReg ? j - 1 : j;
+        const int slot = (head - back < 0) ? head - back + kRing : head - back;
+        const float4 sv = Sb[slot * 64 + lane];
+        const float4 yv = Yb[slot * 64 + lane];
+        sj[0] = sv.x, sj[1] = sv.y, sj[2] = sv.z, sj[3] = sv.w;
+        yj[0] = yv.x, yj[1] = yv.y, yj[2] = yv.z, yj[3] = yv.w;
+      };
       // two-loop recursion in the spectral basis, newest to oldest then back
 #pragma unroll
       for (int r = 0; r < 4; r++) ds[r] = -gs[r];
 #pragma unroll
       for (int j = 0; j < M; j++) {
         if (j < nh) {
-          const int slot = (head - j < 0) ? head - j + M : head - j;
-          const float4 sv = Sb[slot * 64 + lane];
-          const float4 yv = Yb[slot * 64 + lane];
-          const float sj[4] = {sv.x, sv.y, sv.z, sv.w};
+          float sj[4], yj[4];
+          pair(j, sj, yj);
           // the pair added in this step: s.(-g) = -t phi'(t), no reduction
-          al[j] = rho[j] * ((j == 0 && added) ? -tstep * dphi_acc : wave_dot(sj, ds));
-          ds[0] = fmaf(-al[j], yv.x, ds[0]);
-          ds[1] = fmaf(-al[j], yv.y, ds[1]);
-          ds[2] = fmaf(-al[j], yv.z, ds[2]);
-          ds[3] = fmaf(-al[j], yv.w, ds[3]);
+          al[j] = rho[j] * ((j == 0 && added) ? -tstep * dphi_acc
+                            : j == 0         ? wave_dot(sj, ds)
+                                             : wave_dot<true>(sj, ds));
+#pragma unroll
+          for (int r = 0; r < 4; r++) ds[r] = fmaf(-al[j], yj[r], ds[r]);
         }
       }
       if (kCorr && spec_h0 && corr_h0) {
@@ -1390,15 +1500,11 @@ void solve_kernel(WithFrames<SolveArgs> L) {
 #pragma unroll
       for (int j = M - 1; j >= 0; j--) {
         if (j < nh) {
-          const int slot = (head - j < 0) ? head - j + M : head - j;
-          const float4 sv = Sb[slot * 64 + lane];
-          const float4 yv = Yb[slot * 64 + lane];
-          const float yj[4] = {yv.x, yv.y, yv.z, yv.w};
+          float sj[4], yj[4];
+          pair(j, sj, yj);
           const float b = al[j] - rho[j] * wave_dot(yj, ds);
-          ds[0] = fmaf(b, sv.x, ds[0]);
-          ds[1] = fmaf(b, sv.y, ds[1]);
-          ds[2] = fmaf(b, sv.z, ds[2]);
-          ds[3] = fmaf(b, sv.w, ds[3]);
+#pragma unroll
+          for (int r = 0; r < 4; r++) ds[r] = fmaf(b, sj[r], ds[r]);
         }
       }
       step = 1.0f;
@@ -1435,6 +1541,19 @@ void solve_kernel(WithFrames<SolveArgs> L) {
     asm volatile("" : "+v"(ln));
     const int col = ln & 15, grp = ln >> 4;
     const long long ts = F.slot + (t - F.first);
+    if (!PAD && G.r_hi - G.r_lo == 14 && G.c_hi - G.c_lo == 14 && F.os < kRowStride24) {
+      // a window that owns its whole interior (rows and columns 1..14)
+      if (F.out != nullptr) {
+        float *const po = F.out + ((long long)G.bx * F.os + G.by);
+        const unsigned int oo = row_bytes24(grp, F.os) + 4u * (unsigned int)col;
+        if ((unsigned int)(col - 1) < 14u) {
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            if ((r > 0 || grp > 0) && (r < 3 || grp < 3))
+              const_cast<float &>(at_byte(po + (long long)r * F.os, oo)) = u[r];
+        }
+      }
+    } else
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int row = 4 * grp + r;
