@@ -237,6 +237,11 @@ def tile_count(height, width, geometry=GEOM_REFERENCE, window=16):
                                                 int(window)))
 
 
+def _addr(a):
+    """Address of an array's first element."""
+    return a.__array_interface__["data"][0]
+
+
 def _ptr(a):
     return None if a is None else ctypes.c_void_p(a.ctypes.data)
 
@@ -304,9 +309,13 @@ class Context(object):
         frames = (Frame * n)()
         total = 0
         keep = []
+        counts = {}  # tiles of each distinct frame size
+        last_gamma = None
         for i in range(n):
             d = numpy.ascontiguousarray(datas[i], dtype=numpy.float32)
-            g = numpy.ascontiguousarray(gammas[i], dtype=numpy.float32)
+            if gammas[i] is not last_gamma:  # one array for all frames: once
+                last_gamma = gammas[i]
+                g = numpy.ascontiguousarray(last_gamma, dtype=numpy.float32)
             o = outs[i]
             if d.ndim != 2 or g.shape != d.shape or o.shape != d.shape:
                 raise ValueError("frame %d: data, gamma and out must be 2-D of one shape" % i)
@@ -314,19 +323,21 @@ class Context(object):
                 raise ValueError("out arrays must be C-contiguous float32")
             keep += [d, g]
             fr = frames[i]
-            fr.data, fr.gamma, fr.out = d.ctypes.data, g.ctypes.data, o.ctypes.data
-            fr.height, fr.width = d.shape
-            fr.data_stride = fr.gamma_stride = fr.out_stride = 0
+            fr.data, fr.gamma, fr.out = _addr(d), _addr(g), _addr(o)
+            h, w = d.shape
+            geom = int(geometry[i] if hasattr(geometry, "__len__") else geometry)
+            fr.height, fr.width, fr.geometry = h, w, geom
             fr.alpha = float(alphas[i])
-            fr.geometry = int(geometry[i] if hasattr(geometry, "__len__") else geometry)
-            nt = tile_count(fr.height, fr.width, fr.geometry, getattr(self, "window", 16))
+            nt = counts.get((h, w, geom))
+            if nt is None:
+                nt = counts[h, w, geom] = tile_count(h, w, geom, getattr(self, "window", 16))
             if nt < 0:
                 raise ValueError("frame %d of shape %s is too small for this tiling"
                                  % (i, d.shape))
             total += nt
-        iters = numpy.zeros(total, numpy.int32)
-        status = numpy.zeros(total, numpy.int32)
-        cost = numpy.zeros(total, numpy.float32)
+        iters = numpy.empty(total, numpy.int32)
+        status = numpy.empty(total, numpy.int32)
+        cost = numpy.empty(total, numpy.float32)
         check(self.lib.ncs_hip_reduce_frames(self.handle, frames, n, ctypes.byref(params),
                                              _ptr(iters), _ptr(status), _ptr(cost)),
               "ncs_hip_reduce_frames")
@@ -341,7 +352,7 @@ class Context(object):
         if d.ndim != 3 or d.shape[1:] != (r, r) or g.shape != d.shape:
             raise ValueError("tiles must be [n, %d, %d] with matching gamma" % (r, r))
         n = d.shape[0]
-        u = numpy.zeros_like(d)
+        u = numpy.empty_like(d)
         iters = numpy.zeros(n, numpy.int32)
         status = numpy.zeros(n, numpy.int32)
         cost = numpy.zeros(n, numpy.float32)

@@ -90,6 +90,22 @@ struct DevBuf {
   template <class T> T *as() const { return reinterpret_cast<T *>(p); }
 };
 
+// Host-memory batches travel through pinned slots of a fixed size: copies of
+// the caller's (pageable) rows into one slot run beside the DMA of another.
+// hipMemcpy2DAsync from pageable memory, which this replaces, copies row by
+// row at about 25 us each: 13 ms for a 501 x 643 frame, 400 ms for 1000
+// tiles.  A DMA costs some 30 us beside its bytes, so slots are large: a
+// 1000 x 1000 frame takes 1650 us in slots of 128 KB, 660 of 512 KB, 540 of
+// 1 MB.
+constexpr int kStageSlots = 4;
+constexpr size_t kStageSlot = 1 << 20;
+// Batches up to this many bytes (in and out) are not copied to the device:
+// the solve reads and writes the staging memory over PCIe itself.  Call time
+// with copies and without, us: 64 x 80 67 and 36, 200 x 200 85 and 66,
+// 256 x 256 96 and 93, 300 x 300 109 and 116, 400 x 400 168 and 177,
+// 501 x 643 258 and 226.
+constexpr size_t kZeroCopyBytes = kStageSlots * kStageSlot;
+
 // A persistent-solve schedule: history depth, grid, workgroup size and the
 // arithmetic of the basis changes.
 struct Schedule {
@@ -107,7 +123,7 @@ struct ncs_ctx {
   hipStream_t stream = nullptr;
   int cus = 0;
   char arch[64] = {0};
-  DevBuf tables, frames, queue, data, gamma, out, iters, status, cost, tiles_u;
+  DevBuf tables, frames, queue, in, out;
   bool has_mask = false;
   bool general = false;
   int win = 16;  // window side of the reference geometry (the mask's size)
@@ -143,6 +159,10 @@ struct ncs_ctx {
   bool solve_pending = false;
   // device address of the allocation-free entry point's scratch on this GPU
   void *scratch = nullptr;
+  // pinned staging of the host-memory entry points: kStageSlots slots, each
+  // with the event of its last copy
+  char *stage = nullptr;
+  hipEvent_t stage_event[kStageSlots] = {};
 };
 
 // Orders a solve on stream s after the context's previous one.
@@ -264,13 +284,15 @@ extern "C" void ncs_hip_destroy(ncs_ctx *ctx) {
   if (!ctx) return;
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-  DevBuf *bufs[] = {&ctx->tables, &ctx->frames, &ctx->queue, &ctx->data, &ctx->gamma,
-                    &ctx->out, &ctx->iters, &ctx->status, &ctx->cost, &ctx->tiles_u,
+  DevBuf *bufs[] = {&ctx->tables, &ctx->frames, &ctx->queue, &ctx->in, &ctx->out,
                     &ctx->net_params, &ctx->net_packs, &ctx->net_tmp_packs, &ctx->u0_buf};
   for (DevBuf *b : bufs) b->release();
   if (ctx->frames_event) (void)hipEventDestroy(ctx->frames_event);
   if (ctx->solve_done) (void)hipEventDestroy(ctx->solve_done);
   if (ctx->frames_staging) (void)hipHostFree(ctx->frames_staging);
+  if (ctx->stage) (void)hipHostFree(ctx->stage);
+  for (hipEvent_t e : ctx->stage_event)
+    if (e) (void)hipEventDestroy(e);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -320,6 +342,11 @@ extern "C" int ncs_hip_set_otf_mask(ncs_ctx *ctx, const float *mask) {
 extern "C" int ncs_hip_set_otf_mask_window(ncs_ctx *ctx, const float *mask, int win) {
   if (!ctx || !mask) return fail(NCS_E_ARG, "bad arguments");
   if (win < 4 || win > 16 || (win & 1)) return fail(NCS_E_ARG, "window side must be even, 4..16");
+  // the mask the context already holds (programs set it before every call):
+  // its tables stand
+  if (ctx->has_mask && ctx->win == win &&
+      std::memcmp(ctx->mask_fft, mask, (size_t)win * win * sizeof(float)) == 0)
+    return NCS_OK;
   double q[16][16] = {}, qcs[16][16] = {};
   double qmax = 0.0;
   for (int k = 0; k < win; k++)
@@ -333,18 +360,22 @@ extern "C" int ncs_hip_set_otf_mask_window(ncs_ctx *ctx, const float *mask, int 
       qcs[k][l] = 0.5 * (q[k][l] + q[(win - k) % win][(win - l) % win]);
       qmax = std::max(qmax, std::fabs(qcs[k][l]));
     }
+  ctx->has_mask = false;  // until the tables are in place
+  double basis[16][16];
+  for (int a = 0; a < 16; a++)
+    for (int i = 0; i < 16; i++) basis[a][i] = rbasis(a, i, win);
   std::vector<float> &tab = ctx->tab_host;
   double qo_max = 0.0, k_norm = 0.0;
   for (int lane = 0; lane < 64; lane++) {
     int g = lane >> 4, x = lane & 15;
     for (int r = 0; r < 4; r++) {
       int b = 4 * g + r, a = x;
-      tab[lane * kTableLaneFloats + r] = (float)rbasis(x, 4 * g + r, win);
-      tab[lane * kTableLaneFloats + 4 + r] = (float)rbasis(4 * g + r, x, win);
+      tab[lane * kTableLaneFloats + r] = (float)basis[x][4 * g + r];
+      tab[lane * kTableLaneFloats + 4 + r] = (float)basis[4 * g + r][x];
       // FP16 hi/lo pairs of the same entries, each duplicated into both
       // halves of an 8-wide FP16 operand (slots r and 4 + r)
       for (int t = 0; t < 2; t++) {
-        const double v = t == 0 ? rbasis(x, 4 * g + r, win) : rbasis(4 * g + r, x, win);
+        const double v = t == 0 ? basis[x][4 * g + r] : basis[4 * g + r][x];
         uint16_t hi, lo;
         split_f16(v, hi, lo);
         uint16_t *h = reinterpret_cast<uint16_t *>(&tab[lane * kTableLaneFloats + 24 + 8 * t]);
@@ -873,6 +904,106 @@ extern "C" int ncs_hip_solve_tiles_device(ncs_ctx *ctx, const float *data_in,
 // host-memory entry points
 // ---------------------------------------------------------------------------
 
+// Rows of a caller's array: n rows of `row` bytes, `pitch` bytes apart; p may
+// be null for rows that nobody asked for (they are passed over).
+struct HostRows {
+  char *p;
+  size_t row, pitch, n;
+  static HostRows of(const void *p, size_t row, size_t pitch, size_t n) {
+    if (pitch == row) return {static_cast<char *>(const_cast<void *>(p)), row * n, row * n, 1};
+    return {static_cast<char *>(const_cast<void *>(p)), row, pitch, n};
+  }
+};
+
+// Walks a list of rows as one linear run of bytes.
+class RowCursor {
+ public:
+  explicit RowCursor(const std::vector<HostRows> &rows) : v_(rows) {}
+  void gather(char *to, size_t bytes) {
+    walk(bytes, [&](char *p, size_t at, size_t n) { std::memcpy(to + at, p, n); });
+  }
+  void scatter(const char *from, size_t bytes) {
+    walk(bytes, [&](char *p, size_t at, size_t n) { std::memcpy(p, from + at, n); });
+  }
+
+ private:
+  template <class F>
+  void walk(size_t bytes, F f) {
+    for (size_t at = 0; at < bytes;) {
+      const HostRows &r = v_[seg_];
+      const size_t n = std::min(bytes - at, r.row - off_);
+      if (r.p) f(r.p + row_ * r.pitch + off_, at, n);
+      at += n;
+      off_ += n;
+      if (off_ == r.row) {
+        off_ = 0;
+        if (++row_ == r.n) row_ = 0, seg_++;
+      }
+    }
+  }
+  const std::vector<HostRows> &v_;
+  size_t seg_ = 0, row_ = 0, off_ = 0;
+};
+
+static hipError_t stage_ensure(ncs_ctx *ctx) {
+  if (ctx->stage) return hipSuccess;
+  for (hipEvent_t &e : ctx->stage_event)
+    if (!e) {
+      const hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+      if (r != hipSuccess) return r;
+    }
+  void *p = nullptr;
+  const hipError_t r = hipHostMalloc(&p, kStageSlots * kStageSlot, hipHostMallocDefault);
+  if (r == hipSuccess) ctx->stage = static_cast<char *>(p);
+  return r;
+}
+
+// Enqueues the rows' upload to `dst`, slot by slot.  Every slot is free when
+// it starts (each host call waits for the stream before it returns) and its
+// copies may still be running when it returns.
+static hipError_t upload_rows(ncs_ctx *ctx, const std::vector<HostRows> &rows, char *dst,
+                              size_t bytes, hipStream_t s) {
+  RowCursor cur(rows);
+  hipError_t e = hipSuccess;
+  int k = 0;
+  for (size_t at = 0; at < bytes && e == hipSuccess; at += kStageSlot, k++) {
+    const int slot = k % kStageSlots;
+    if (k >= kStageSlots) e = hipEventSynchronize(ctx->stage_event[slot]);
+    if (e != hipSuccess) break;
+    char *buf = ctx->stage + slot * kStageSlot;
+    const size_t n = std::min(kStageSlot, bytes - at);
+    cur.gather(buf, n);
+    e = hipMemcpyAsync(dst + at, buf, n, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipEventRecord(ctx->stage_event[slot], s);
+  }
+  return e;
+}
+
+// Downloads `bytes` from `src` into the rows: the copies run a ring of slots
+// ahead of the host, which returns with every row written.
+static hipError_t download_rows(ncs_ctx *ctx, const std::vector<HostRows> &rows, const char *src,
+                                size_t bytes, hipStream_t s) {
+  RowCursor cur(rows);
+  const size_t pieces = (bytes + kStageSlot - 1) / kStageSlot;
+  hipError_t e = hipSuccess;
+  auto piece = [&](size_t k) { return std::min(kStageSlot, bytes - k * kStageSlot); };
+  auto enqueue = [&](size_t k) {
+    const int slot = (int)(k % kStageSlots);
+    hipError_t r = hipMemcpyAsync(ctx->stage + slot * kStageSlot, src + k * kStageSlot, piece(k),
+                                  hipMemcpyDeviceToHost, s);
+    return r == hipSuccess ? hipEventRecord(ctx->stage_event[slot], s) : r;
+  };
+  for (size_t k = 0; k < pieces && k < (size_t)kStageSlots && e == hipSuccess; k++) e = enqueue(k);
+  for (size_t k = 0; k < pieces && e == hipSuccess; k++) {
+    const int slot = (int)(k % kStageSlots);
+    e = hipEventSynchronize(ctx->stage_event[slot]);
+    if (e != hipSuccess) break;
+    cur.scatter(ctx->stage + slot * kStageSlot, piece(k));
+    if (k + kStageSlots < pieces) e = enqueue(k + kStageSlots);
+  }
+  return e;
+}
+
 extern "C" int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int n_frames,
                                      const ncs_params *params, int *iterations,
                                      int *status, float *cost) {
@@ -892,67 +1023,81 @@ extern "C" int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int 
   HIPCHK(set_device(ctx));
   hipStream_t s = ctx->stream;
   HIPCHK(order_after_previous(ctx, s));
-  // device layout: each frame's data / out packed [H][W]; gamma deduplicated
-  size_t pix = 0, gpix = 0;
-  std::vector<size_t> off(n_frames), goff(n_frames);
-  std::vector<int> gsrc(n_frames, -1);
-  for (int i = 0; i < n_frames; i++) {
-    off[i] = pix;
-    pix += (size_t)frames[i].height * frames[i].width;
-    for (int j = 0; j < i; j++)
-      if (frames[j].gamma == frames[i].gamma && frames[j].height == frames[i].height &&
-          frames[j].width == frames[i].width &&
-          fd[j].gs == fd[i].gs) { gsrc[i] = j; break; }
-    if (gsrc[i] < 0) {
-      goff[i] = gpix;
-      gpix += (size_t)frames[i].height * frames[i].width;
-    } else {
-      goff[i] = goff[gsrc[i]];
-    }
-  }
-  HIPCHK(ctx->data.ensure(pix * 4));
-  HIPCHK(ctx->out.ensure(pix * 4));
-  HIPCHK(ctx->gamma.ensure(gpix * 4));
-  HIPCHK(ctx->iters.ensure(total * 4));
-  HIPCHK(ctx->status.ensure(total * 4));
-  HIPCHK(ctx->cost.ensure(total * 4));
-  float *dd = ctx->data.as<float>(), *dg = ctx->gamma.as<float>(), *dout = ctx->out.as<float>();
+  // Device layout, one linear region each way: in = every frame's data, then
+  // the distinct gammas, packed [H][W]; out = every frame's image, then the
+  // per-tile results that are asked for.
+  std::vector<HostRows> in, out;
+  size_t in_bytes = 0, out_bytes = 0;
+  std::vector<size_t> d_off(n_frames), g_off(n_frames), o_off(n_frames);
+  auto add = [](std::vector<HostRows> &v, size_t &at, const void *p, size_t row, size_t pitch,
+                size_t rows) {
+    const size_t here = at;
+    at += row * rows;
+    v.push_back(HostRows::of(p, row, pitch, rows));
+    return here;
+  };
   for (int i = 0; i < n_frames; i++) {
     const ncs_frame &f = frames[i];
-    HIPCHK(hipMemcpy2DAsync(dd + off[i], f.width * 4, f.data, fd[i].ds * 4, f.width * 4,
-                            f.height, hipMemcpyHostToDevice, s));
-    if (gsrc[i] < 0)
-      HIPCHK(hipMemcpy2DAsync(dg + goff[i], f.width * 4, f.gamma, fd[i].gs * 4, f.width * 4,
-                              f.height, hipMemcpyHostToDevice, s));
-    fd[i].data = dd + off[i];
-    fd[i].gamma = dg + goff[i];
-    fd[i].out = f.out ? dout + off[i] : nullptr;
-    fd[i].ds = fd[i].gs = fd[i].os = f.width;
+    d_off[i] = add(in, in_bytes, f.data, f.width * 4ull, fd[i].ds * 4ull, f.height);
+    o_off[i] = add(out, out_bytes, f.out, f.width * 4ull, fd[i].os * 4ull, f.height);
+  }
+  for (int i = 0; i < n_frames; i++) {
+    const ncs_frame &f = frames[i];
+    int same = -1;
+    for (int j = 0; j < i && same < 0; j++)
+      if (frames[j].gamma == f.gamma && frames[j].height == f.height &&
+          frames[j].width == f.width && fd[j].gs == fd[i].gs)
+        same = j;
+    g_off[i] = same >= 0 ? g_off[same]
+                         : add(in, in_bytes, f.gamma, f.width * 4ull, fd[i].gs * 4ull, f.height);
+  }
+  size_t r_off[3] = {};
+  const void *const results[3] = {iterations, status, cost};
+  for (int k = 0; k < 3; k++)
+    if (results[k]) r_off[k] = add(out, out_bytes, results[k], total * 4ull, total * 4ull, 1);
+
+  HIPCHK(stage_ensure(ctx));
+  const bool direct = in_bytes + out_bytes <= kZeroCopyBytes;
+  char *d_in, *d_out;
+  if (direct) {
+    void *dev = nullptr;
+    HIPCHK(hipHostGetDevicePointer(&dev, ctx->stage, 0));
+    d_in = static_cast<char *>(dev);
+    d_out = d_in + in_bytes;
+    RowCursor(in).gather(ctx->stage, in_bytes);
+  } else {
+    HIPCHK(ctx->in.ensure(in_bytes));
+    HIPCHK(ctx->out.ensure(out_bytes));
+    d_in = ctx->in.as<char>();
+    d_out = ctx->out.as<char>();
+  }
+  for (int i = 0; i < n_frames; i++) {
+    fd[i].data = reinterpret_cast<float *>(d_in + d_off[i]);
+    fd[i].gamma = reinterpret_cast<float *>(d_in + g_off[i]);
+    fd[i].out = frames[i].out ? reinterpret_cast<float *>(d_out + o_off[i]) : nullptr;
+    fd[i].ds = fd[i].gs = fd[i].os = frames[i].width;
   }
   schedule_small_first(fd, total);
-  const FrameDev *table = nullptr;
-  rc = upload_frames(ctx, fd, s, &table);
+  const bool pad = any_pad(ctx, frames, n_frames);
+  hipError_t e = direct ? hipSuccess : upload_rows(ctx, in, d_in, in_bytes, s);
+  if (e == hipSuccess) {
+    const FrameDev *table = nullptr;
+    rc = upload_frames(ctx, fd, s, &table);
+    if (rc == NCS_OK)
+      rc = enqueue_solve(ctx, table, fd.data(), n_frames, pad, total, params, nullptr,
+                         iterations ? reinterpret_cast<int *>(d_out + r_off[0]) : nullptr,
+                         status ? reinterpret_cast<int *>(d_out + r_off[1]) : nullptr,
+                         cost ? reinterpret_cast<float *>(d_out + r_off[2]) : nullptr,
+                         ctx->queue.as<unsigned int>(), s);
+    if (rc == NCS_OK && !direct) e = download_rows(ctx, out, d_out, out_bytes, s);
+    if (rc == NCS_OK && e == hipSuccess) e = mark_solve(ctx, s);
+  }
+  // whatever was enqueued is complete before the caller's memory is let go
+  const hipError_t e2 = hipStreamSynchronize(s);
   if (rc) return rc;
-  rc = enqueue_solve(ctx, table, fd.data(), n_frames, any_pad(ctx, frames, n_frames), total,
-                     params, nullptr, ctx->iters.as<int>(), ctx->status.as<int>(),
-                     ctx->cost.as<float>(), ctx->queue.as<unsigned int>(), s);
-  if (rc) {
-    (void)hipStreamSynchronize(s);
-    return rc;
-  }
-  for (int i = 0; i < n_frames; i++) {
-    const ncs_frame &f = frames[i];
-    if (!f.out) continue;
-    int os = f.out_stride > 0 ? f.out_stride : f.width;
-    HIPCHK(hipMemcpy2DAsync(f.out, os * 4, dout + off[i], f.width * 4, f.width * 4, f.height,
-                            hipMemcpyDeviceToHost, s));
-  }
-  if (iterations)
-    HIPCHK(hipMemcpyAsync(iterations, ctx->iters.p, total * 4, hipMemcpyDeviceToHost, s));
-  if (status) HIPCHK(hipMemcpyAsync(status, ctx->status.p, total * 4, hipMemcpyDeviceToHost, s));
-  if (cost) HIPCHK(hipMemcpyAsync(cost, ctx->cost.p, total * 4, hipMemcpyDeviceToHost, s));
-  HIPCHK(mark_solve(ctx, s));
-  HIPCHK(hipStreamSynchronize(s));
+  HIPCHK(e);
+  HIPCHK(e2);
+  if (direct) RowCursor(out).scatter(ctx->stage + in_bytes, out_bytes);
   return NCS_OK;
 }
 

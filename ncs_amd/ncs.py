@@ -43,7 +43,11 @@ NCSCUDAException = NCSHipException
 def checkOTFMask(otf_mask):
     """Symmetry test of opencl/pyOpenCLNCS/ncs.py:225-233 (and
     clib/pyCNCS/ncs_c.py:239-247): max(imag(ifft2(fftshift(M)))) <= 1e-12."""
-    otf_mask_fft = numpy.fft.ifft2(numpy.fft.fftshift(otf_mask))
+    return _symmetric(numpy.fft.fftshift(otf_mask))
+
+
+def _symmetric(otf_mask_fft_order):
+    otf_mask_fft = numpy.fft.ifft2(otf_mask_fft_order)
     return not (numpy.max(numpy.imag(otf_mask_fft)) > 1.0e-12)
 
 
@@ -85,11 +89,12 @@ class NCSHip(object):
                 raise NCSHipException("OTF must be square!")
             if otf_mask.size != self.size * self.size:
                 raise NCSHipException("OTF size must match sub-region size!")
-            if not checkOTFMask(otf_mask):
-                raise NCSHipException("OTF does not have the expected symmetry!")
         elif otf_mask.shape != (self.size, self.size):
             raise NCSHipException("OTF size must match sub-region size!")
-        self.otf_mask = numpy.fft.fftshift(otf_mask).astype(numpy.float32)
+        shifted = numpy.fft.fftshift(otf_mask)
+        if self.strict and not _symmetric(shifted):
+            raise NCSHipException("OTF does not have the expected symmetry!")
+        self.otf_mask = shifted.astype(numpy.float32)
 
     def reduceNoise(self, images, alpha, verbose=False, geometry="reference",
                     return_info=False):
@@ -119,8 +124,9 @@ class NCSHip(object):
             if geom == _lib.GEOM_REFERENCE and min(im.shape) < self.size - 2:
                 raise NCSHipException("images must be at least %d pixels on each side"
                                       % (self.size - 2))
-            datas.append(im.astype(numpy.float32))
-            outs.append(numpy.zeros(im.shape, dtype=numpy.float32))
+            datas.append(numpy.asarray(im, dtype=numpy.float32))
+            # (every pixel is owned by one window, so the solve writes them all)
+            outs.append(numpy.empty(im.shape, dtype=numpy.float32))
         self.ctx.set_otf_mask(self.otf_mask)
         iters, status, cost = self.ctx.reduce_frames(datas, gammas, outs, alphas, geom,
                                                      self.params)
@@ -160,7 +166,10 @@ def reduceNoise(images, gamma, otf_mask, alpha, strict=True, verbose=False, *,
     return_info=True)."""
     ncs = NCSHip(strict=strict, device=device, params=params)
     ncs.setOTFMask(otf_mask)
-    ncs.setGamma(gamma)
+    if isinstance(gamma, (list, tuple)):
+        ncs.setGamma(gamma)
+    else:  # used within this call: no copy of a float32 map
+        ncs.gamma = numpy.asarray(gamma, dtype=numpy.float32)
     return ncs.reduceNoise(images, alpha, verbose=verbose, geometry=geometry,
                            return_info=return_info)
 
