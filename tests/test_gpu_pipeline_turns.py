@@ -22,8 +22,8 @@ def _pinned(dtype, fill=None):
     return a
 
 
-def _line(ctx, gamma, **kw):
-    pl = _lib.Pipeline(ctx, [SHAPE], [0.1], params=_lib.default_params(**kw))
+def _line(ctx, gamma, history=5):
+    pl = _lib.Pipeline(ctx, [SHAPE], [0.1], params=_lib.default_params(history=history))
     pl.set_gamma(0, gamma)
     return pl
 
@@ -40,7 +40,7 @@ def test_images_are_those_of_a_pipeline_alone(gpu_ctx, mode):
     alone = _line(gpu_ctx, gamma)
     for a, b in zip(ins, want):
         alone.wait(alone.launch([a], [b]))
-    lines = [_line(gpu_ctx, gamma), _line(gpu_ctx, gamma, history=2 if mode == "other" else 0)]
+    lines = [_line(gpu_ctx, gamma), _line(gpu_ctx, gamma, 2 if mode == "other" else 5)]
     if mode == "other":
         want[1::2] = [_pinned(torch.float32) for _ in want[1::2]]
         for a, b in zip(ins[1::2], want[1::2]):
