@@ -106,6 +106,7 @@ struct SolveArgs {
   long long total_tiles;
   TileSchedule sched;          // filled in by launch_solve
   unsigned int *queue;         // kQueues work-queue counters (kQueueBytes)
+  unsigned int *queue_next;    // the next solve's, cleared by this one (or nullptr)
   const float *tables;         // [64][16] per-lane OTF/DFT tables
   const float *u0;             // [tiles][256] warm start or nullptr
   int *iterations;             // [tiles] or nullptr

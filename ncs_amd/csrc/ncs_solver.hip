@@ -933,6 +933,10 @@ void solve_kernel(WithFrames<SolveArgs> L) {
     next = w * A0.sched.per_wave + min(w, A0.sched.extra);
     end = next + A0.sched.per_wave + (w < A0.sched.extra ? 1u : 0u);
   }
+  // the next solve's counters: idle now, since solves that take turns with
+  // them run one after the other
+  if (blockIdx.x == 0 && threadIdx.x < kQueues && A0.queue_next != nullptr)
+    A0.queue_next[threadIdx.x * kQueueStride] = 0u;
   int qv = 0;  // dynamic ranges found exhausted
   auto next_tile = [&]() -> long long {
     if (next < end) return (long long)(next++);
@@ -1725,6 +1729,8 @@ int solve_waves_per_cu(int m, bool general, bool pad, bool f16, int wpg) {
 // Launches `waves` persistent waves in workgroups of `wpg` waves (waves is
 // rounded up to a multiple of wpg).  Without a device frame table (a.frames
 // null) the a.n_frames <= kInlineFrames frames are at inline_frames (host).
+// `clean`: the counters at a.queue are zero; else a kernel resets them first,
+// where the launch needs them.
 //
 // Shares of the tiles.  A device-scope atomic is resolved beyond the XCD's
 // L2, so tiles are assigned statically where that balances: up to
@@ -1739,7 +1745,7 @@ int solve_waves_per_cu(int m, bool general, bool pad, bool f16, int wpg) {
 // 120 and 87 us, 150 and 128 us.  Chunks of two or three were within 1% with
 // the linear start's short tiles and 2% slower with the plain start's.
 hipError_t launch_solve(int m, bool general, bool pad, bool f16, unsigned int waves, int wpg,
-                        hipStream_t s, SolveArgs a, const FrameDev *inline_frames) {
+                        hipStream_t s, SolveArgs a, const FrameDev *inline_frames, bool clean) {
   SolveKernelFn fn = solve_kernel_for(m, general, pad, f16);
   if (!fn || wpg < 1 || wpg > kMaxWavesPerGroup || waves == 0) return hipErrorInvalidValue;
   const unsigned int groups = (waves + wpg - 1) / wpg;
@@ -1753,7 +1759,7 @@ hipError_t launch_solve(int m, bool general, bool pad, bool f16, unsigned int wa
     a.sched.per_wave = (unsigned int)(a.total_tiles * 2 / 5 / n_waves);
     a.sched.extra = 0;
     a.sched.dyn0 = (unsigned int)(a.sched.per_wave * n_waves);
-    hipLaunchKernelGGL(reset_queue_kernel, dim3(1), dim3(64), 0, s, a.queue);
+    if (!clean) hipLaunchKernelGGL(reset_queue_kernel, dim3(1), dim3(64), 0, s, a.queue);
   }
   WithFrames<SolveArgs> L;
   L.args = a;
