@@ -192,15 +192,17 @@ __device__ __forceinline__ void store_row_std(__bf16 *dst, int y, int lane, i4 v
 }
 
 // Layer 1 (2 -> 32 channels), K = tap * 2 + cin padded to 32.  The inputs sit
-// in LDS as an 18 x 18 grid of (x0, x1) float pairs with a zero border, so
-// lane (g, x) reads its K = 8g..8g+7 (taps 4g..4g+3) of row y as four float2
+// in LDS as an 18 x 18 grid of (x0, x1) BF16 pairs with a zero border, so
+// lane (g, x) reads its K = 8g..8g+7 (taps 4g..4g+3) of row y as four pairs
 // at fixed offsets; taps past 8 read the zero border column of the row.
+// Rounded once when it is written, a pair is not converted again for each of
+// the nine taps that read it.
 __device__ __forceinline__ int in_pad_offset(int tap, int x) {
-  return tap < 9 ? ((tap / 3) * 18 + x + tap % 3) * 2 : 0;
+  return tap < 9 ? (tap / 3) * 18 + x + tap % 3 : 0;
 }
 
 template <class Keep>
-__device__ __forceinline__ void layer_in2(const float *in_pad, const i4 *packs,
+__device__ __forceinline__ void layer_in2(const int *in_pad, const i4 *packs,
                                           const float *bias, int lane, i4 (&act)[16],
                                           Keep keep) {
   const i4 A0 = packs[lane], A1 = packs[64 + lane];
@@ -213,10 +215,7 @@ __device__ __forceinline__ void layer_in2(const float *in_pad, const i4 *packs,
   for (int y = 0; y < 16; y++) {
     i4 B;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const float2 v = *reinterpret_cast<const float2 *>(in_pad + y * 36 + off[j]);
-      B[j] = bf16_pair(v.x, v.y);
-    }
+    for (int j = 0; j < 4; j++) B[j] = in_pad[y * 18 + off[j]];
     act[y] = relu_row(mfma_bf16(A0, B, c0), mfma_bf16(A1, B, c1));
     keep(y, act[y]);
   }
@@ -289,81 +288,118 @@ __device__ __forceinline__ void layer32(i4 (&act)[16], const i4 *packs_in, const
 // (g, x) holds A[x][8g..8g+7] (pixel x, K chunk g), and B_dy[k][n] =
 // W4[fwd_channel(k)][dy][n] for n = dx < 3.  Three chained MFMA per row give
 // D_y[x'][n] = sum_dy sum_ci a3[ci][y + dy - 1][x'] W4[ci][dy][n] (D lane
-// (g, n) holds x' = 4g..4g+3); all 16 rows go to dbuf ([16][16][3] FP32 LDS)
-// and, after one barrier,
+// (g, n) holds x' = 4g..4g+3); all 16 rows go to dbuf (three FP32 planes
+// [16][16] in LDS, kOutPlane apart so that the planes' writes use different
+// banks) and, after one barrier,
 //   out[y][x] = b4 + D_y[x - 1][0] + D_y[x][1] + D_y[x + 1][2]
 // (zero past the tile) for the pixels (4g + r, x) of lane (g, x), r = 0..3.
+constexpr int kOutPlane = 256 + 16;
 __device__ __forceinline__ f4 layer_out1(const i4 (&act)[16], const i4 *packs,
                                          float *dbuf, float b4, int lane) {
   const i4 B0 = packs[lane], B1 = packs[64 + lane], B2 = packs[128 + lane];
   const int n = lane & 15, g = lane >> 4;
+  f4 d[16];
 #pragma unroll
   for (int y = 0; y < 16; y++) {
-    f4 d = {0.f, 0.f, 0.f, 0.f};
-    if (y > 0) d = mfma_bf16(act[y - 1], B0, d);
-    d = mfma_bf16(act[y], B1, d);
-    if (y < 15) d = mfma_bf16(act[y + 1], B2, d);
-    if (n < 3)
-#pragma unroll
-      for (int r = 0; r < 4; r++) dbuf[(y * 16 + 4 * g + r) * 3 + n] = d[r];
+    d[y] = (f4){0.f, 0.f, 0.f, 0.f};
+    if (y > 0) d[y] = mfma_bf16(act[y - 1], B0, d[y]);
+    d[y] = mfma_bf16(act[y], B1, d[y]);
+    if (y < 15) d[y] = mfma_bf16(act[y + 1], B2, d[y]);
   }
+  if (n < 3)
+#pragma unroll
+    for (int y = 0; y < 16; y++)
+      *reinterpret_cast<f4 *>(dbuf + n * kOutPlane + y * 16 + 4 * g) = d[y];
   wave_sync();
+  const int nl = n > 0 ? n - 1 : 0, nr = n < 15 ? n + 1 : 15;
   f4 out;
 #pragma unroll
   for (int r = 0; r < 4; r++) {
-    const float *D = dbuf + (4 * g + r) * 48;
-    float v = b4 + D[n * 3 + 1];
-    if (n > 0) v += D[(n - 1) * 3 + 0];
-    if (n < 15) v += D[(n + 1) * 3 + 2];
+    const float *D = dbuf + (4 * g + r) * 16;
+    const float l = D[nl], c = D[kOutPlane + n], rr = D[2 * kOutPlane + nr];
+    float v = b4 + c;
+    v += n > 0 ? l : 0.0f;
+    v += n < 15 ? rr : 0.0f;
     out[r] = v;
   }
   return out;
 }
 
-// Writes the zero border of the 18 x 18 input grid (68 cells).
-__device__ __forceinline__ void in_pad_border(float *in_pad, int lane) {
+// Writes the zero border of the 18 x 18 input grid (68 cells); the tiles
+// write the inside only.
+__device__ __forceinline__ void in_pad_border(int *in_pad, int lane) {
   for (int c = lane; c < 68; c += 64) {
     int cell;
     if (c < 18) cell = c;                          // top row
     else if (c < 36) cell = 17 * 18 + (c - 18);    // bottom row
     else if (c < 52) cell = (c - 35) * 18;         // left column, rows 1..16
     else cell = (c - 51) * 18 + 17;                // right column, rows 1..16
-    *reinterpret_cast<float2 *>(in_pad + 2 * cell) = make_float2(0.0f, 0.0f);
+    in_pad[cell] = 0;
   }
 }
 
-__device__ __forceinline__ void in_pad_put(float *in_pad, int row, int col, float x0, float x1) {
-  *reinterpret_cast<float2 *>(in_pad + 2 * ((row + 1) * 18 + col + 1)) = make_float2(x0, x1);
+__device__ __forceinline__ void in_pad_put(int *in_pad, int row, int col, float x0, float x1) {
+  in_pad[(row + 1) * 18 + col + 1] = bf16_pair(x0, x1);
+}
+
+// a and b summed over the wave (uniform), lanes 32, 16, 8, 4, 2 and 1 apart:
+// row swaps and DPP, where __shfl_xor would take twelve LDS round trips.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __int_as_float(
+                 __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ void wave_sum2(float &a, float &b) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b),
+                                                  false, false);
+  float s = __uint_as_float(p[0]) + __uint_as_float(p[1]);  // a below lane 32, b above
+  const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(s), __float_as_uint(s),
+                                                  false, false);
+  s = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+  s = dpp_add<0x128>(s);  // row_ror:8
+  s = dpp_add<0x124>(s);  // row_ror:4 (equal 8 lanes apart by now)
+  s = dpp_add<0x4E>(s);   // quad_perm [2, 3, 0, 1]
+  s = dpp_add<0xB1>(s);   // quad_perm [1, 0, 3, 2]
+  a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), 0));
+  b = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), 32));
 }
 
 // Normalises one tile held in the solver's lane layout (lane (g, x) has
 // rows 4g + r, column x) into the padded input grid; returns sigma.
 __device__ __forceinline__ void tile_inputs(const float *d_tile_lane, const float *gm_lane,
-                                            float *in_pad, int lane, float &sigma) {
-  float red[2] = {d_tile_lane[0] + d_tile_lane[1] + (d_tile_lane[2] + d_tile_lane[3]),
-                  gm_lane[0] + gm_lane[1] + (gm_lane[2] + gm_lane[3])};
-  for (int off = 32; off >= 1; off >>= 1) {
-    red[0] += __shfl_xor(red[0], off);
-    red[1] += __shfl_xor(red[1], off);
-  }
-  const float mu = red[0] * (1.0f / 256.0f), gmean = red[1] * (1.0f / 256.0f);
+                                            int *in_pad, int lane, float &sigma) {
+  float mu = d_tile_lane[0] + d_tile_lane[1] + (d_tile_lane[2] + d_tile_lane[3]);
+  float gmean = gm_lane[0] + gm_lane[1] + (gm_lane[2] + gm_lane[3]);
+  wave_sum2(mu, gmean);
+  mu *= 1.0f / 256.0f;
+  gmean *= 1.0f / 256.0f;
   sigma = sqrtf(fmaxf(mu, 1.0f) + gmean);
   const float inv = 1.0f / sigma;
   const int x = lane & 15, g = lane >> 4;
-  in_pad_border(in_pad, lane);
 #pragma unroll
   for (int r = 0; r < 4; r++)
     in_pad_put(in_pad, 4 * g + r, x, (d_tile_lane[r] - mu) * inv, gm_lane[r] * inv * inv);
 }
 
-// The network body on one tile whose inputs are in the padded grid `io`
-// (18 x 18 float pairs, then reused as layer 4's [16][16][3] partial sums);
-// returns the output y at pixels (4g + r, x) of lane (g, x).  pk / bl: the
-// forward packs and biases staged in LDS.  acts (may be NULL): post-ReLU
-// layer 1-3 activations, BF16 [3][n][256][32] in the standard channel order,
-// of tile t.  One wave runs it; io is the wave's own.
-__device__ __forceinline__ f4 net_body(float *io, const i4 *pk, const float *bl, int lane,
-                                       __bf16 *acts, long long n, long long t) {
+// A wave's LDS: the padded input grid (18 x 18 BF16 pairs), layer 4's partial
+// sums and the tile's data.
+constexpr int kNetGridInts = 18 * 18;
+constexpr int kNetOutFloats = 3 * kOutPlane;
+constexpr int kNetWaveFloats = kNetGridInts + kNetOutFloats + 256;
+static_assert(kNetGridInts % 4 == 0 && kNetWaveFloats % 4 == 0, "16-byte rows of dbuf");
+
+// The network body on one tile whose inputs are in the padded grid; returns
+// the output y at pixels (4g + r, x) of lane (g, x).  pk / bl: the forward
+// packs and biases staged in LDS.  acts (may be NULL): post-ReLU layer 1-3
+// activations, BF16 [3][n][256][32] in the standard channel order, of tile t.
+// One wave runs it; the grid and dbuf are the wave's own.  before_out() runs
+// before layer 4: loads of the next tile are issued there, where the middle
+// layers' weights have left their registers and three matrix products a row
+// cover the loads' way.
+template <class BeforeOut>
+__device__ __forceinline__ f4 net_body(const int *grid, float *dbuf, const i4 *pk,
+                                       const float *bl, int lane, __bf16 *acts, long long n,
+                                       long long t, BeforeOut before_out) {
   auto keep = [&](int layer) {
     return [=](int y, i4 v) {
       if (acts != nullptr)
@@ -373,20 +409,17 @@ __device__ __forceinline__ f4 net_body(float *io, const i4 *pk, const float *bl,
   const int z = opaque_zero();
   i4 act[16];
   wave_sync();  // the input grid is complete
-  layer_in2(io, pk + (PK_L1 - PK_L1) * 64 + z, bl + z, lane, act, keep(0));
+  layer_in2(grid, pk + (PK_L1 - PK_L1) * 64 + z, bl + z, lane, act, keep(0));
   layer32(act, pk + (PK_L2 - PK_L1) * 64, bl + 32, lane, keep(1));
   layer32(act, pk + (PK_L3 - PK_L1) * 64, bl + 64, lane, keep(2));
-  wave_sync();  // every read of the grid precedes layer 4's writes over it
-  return layer_out1(act, pk + (PK_L4T - PK_L1) * 64 + z, io, bl[96 + z], lane);
+  before_out();
+  return layer_out1(act, pk + (PK_L4T - PK_L1) * 64 + z, dbuf, bl[96 + z], lane);
 }
 
 // Forward workgroups: kNetWaves waves, each running its own tiles, share the
-// forward packs (layers 1-4, 41 KB) and biases staged once in LDS; each
-// wave owns an input grid / layer-4 buffer and a copy of its tile's data.
+// forward packs (layers 1-4, 41 KB) and biases staged once in LDS.
 constexpr int kNetWaves = 4;
 constexpr int kFwdPacks = PK_B4 - PK_L1;
-constexpr int kNetIoFloats = 768;  // max(18 * 18 * 2, 16 * 16 * 3)
-constexpr int kNetWaveFloats = kNetIoFloats + 256;
 constexpr int kNetFwdLdsBytes = kFwdPacks * 1024 + 128 * 4 + kNetWaves * kNetWaveFloats * 4;
 
 // Copies the forward packs and the biases [b1 | b2 | b3 | b4] into LDS.
@@ -411,15 +444,16 @@ void net_fwd_kernel(const float *__restrict__ xin, float *__restrict__ yout,
   // the wave index is uniform: read it into a scalar register so the tile
   // loop's index arithmetic and frame-table reads stay on the scalar unit
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  float *io = bl + 128 + wave * kNetWaveFloats;
+  int *const grid = reinterpret_cast<int *>(bl + 128 + wave * kNetWaveFloats);
+  float *const dbuf = reinterpret_cast<float *>(grid + kNetGridInts);
   const int col = lane & 15, grp = lane >> 4;
   stage_forward(packs, P, pk, bl);
+  in_pad_border(grid, lane);
   for (long long t = (long long)blockIdx.x * kNetWaves + wave; t < n;
        t += (long long)gridDim.x * kNetWaves) {
-    in_pad_border(io, lane);
     for (int i = lane; i < 256; i += 64)
-      in_pad_put(io, i >> 4, i & 15, xin[t * 512 + i], xin[t * 512 + 256 + i]);
-    const f4 y = net_body(io, pk, bl, lane, acts, n, t);
+      in_pad_put(grid, i >> 4, i & 15, xin[t * 512 + i], xin[t * 512 + 256 + i]);
+    const f4 y = net_body(grid, dbuf, pk, bl, lane, acts, n, t, [] {});
 #pragma unroll
     for (int r = 0; r < 4; r++) yout[t * 256 + (4 * grp + r) * 16 + col] = y[r];
     wave_sync();
@@ -431,7 +465,6 @@ void net_fwd_kernel(const float *__restrict__ xin, float *__restrict__ yout,
 __global__ __launch_bounds__(64 * kNetWaves) __attribute__((amdgpu_waves_per_eu(2)))
 void net_warm_kernel(WithFrames<NetWarmArgs> W) {
   const long long total = W.args.total;
-  float *__restrict__ u0 = W.args.u0;
   const i4 *__restrict__ packs = reinterpret_cast<const i4 *>(W.args.packs);
   const float *__restrict__ P = W.args.params;
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -441,12 +474,19 @@ void net_warm_kernel(WithFrames<NetWarmArgs> W) {
   // loop's index arithmetic and frame-table reads stay on the scalar unit
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const FrameConst *fc = frame_table<NetWarmArgs>(W.args.frames);
-  float *io = bl + 128 + wave * kNetWaveFloats;
-  float *dkeep = io + kNetIoFloats;
+  int *const grid = reinterpret_cast<int *>(bl + 128 + wave * kNetWaveFloats);
+  float *const dbuf = reinterpret_cast<float *>(grid + kNetGridInts);
+  float *const dkeep = dbuf + kNetOutFloats;
   const int col = lane & 15, grp = lane >> 4;
-  stage_forward(packs, P, pk, bl);
-  for (long long t = (long long)blockIdx.x * kNetWaves + wave; t < total;
-       t += (long long)gridDim.x * kNetWaves) {
+
+  // Tile t's window, edge-clamped in the reference geometry and zero-padded
+  // in blocks, and the place of its start.  Both read the clamped pixel (32-bit
+  // offsets from uniform pointers: the host keeps every frame below 2^31
+  // elements), so that the eight loads go out together.
+  auto load = [&](long long t, float (&d)[4], float (&gm)[4]) -> float * {
+    int ln = lane;  // formed here: held across the layers it would be spilled
+    asm volatile("" : "+v"(ln));
+    const int col = ln & 15, grp = ln >> 4;
     int lo = 0, hi = W.args.n_frames - 1;
     while (lo < hi) {
       int mid = (lo + hi + 1) >> 1;
@@ -456,39 +496,44 @@ void net_warm_kernel(WithFrames<NetWarmArgs> W) {
     const int local = (int)(t - F.first);  // a frame has fewer than 2^31 windows
     const int a = (int)div_by((unsigned int)local, (unsigned int)F.ty, F.ty_magic);
     const int b = local - a * F.ty;
-    int bx, by, hv = 16, wv = 16;
-    if (F.geom == NCS_GEOM_REFERENCE) {
-      bx = min(-1 + 14 * a, F.H - 15);
-      by = min(-1 + 14 * b, F.W - 15);
-    } else {
-      bx = 16 * a;
-      by = 16 * b;
-      hv = min(16, F.H - bx);
-      wv = min(16, F.W - by);
-    }
-    float d[4], gm[4];
+    const bool ref = F.geom == NCS_GEOM_REFERENCE;
+    const int bx = ref ? min(-1 + 14 * a, F.H - 15) : 16 * a;
+    const int by = ref ? min(-1 + 14 * b, F.W - 15) : 16 * b;
+    const unsigned int gc = (unsigned int)min(max(by + col, 0), F.W - 1);
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int row = 4 * grp + r;
-      // 32-bit element offsets from the uniform base pointers (the host keeps
-      // every frame below 2^31 elements)
-      if (F.geom == NCS_GEOM_REFERENCE) {
-        const int gr = min(max(bx + row, 0), F.H - 1), gc = min(max(by + col, 0), F.W - 1);
-        d[r] = F.data[(unsigned int)(gr * F.ds + gc)];
-        gm[r] = F.gamma[(unsigned int)(gr * F.gs + gc)];
-      } else {
-        const bool ok = row < hv && col < wv;
-        d[r] = ok ? F.data[(unsigned int)((bx + row) * F.ds + by + col)] : 0.0f;
-        gm[r] = ok ? F.gamma[(unsigned int)((bx + row) * F.gs + by + col)] : 0.0f;
+      const unsigned int gr = (unsigned int)min(max(bx + 4 * grp + r, 0), F.H - 1);
+      d[r] = F.data[gr * (unsigned int)F.ds + gc];
+      gm[r] = F.gamma[gr * (unsigned int)F.gs + gc];
+    }
+    if (!ref) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const bool ok = bx + 4 * grp + r < F.H && by + col < F.W;
+        d[r] = ok ? d[r] : 0.0f;
+        gm[r] = ok ? gm[r] : 0.0f;
       }
     }
+    // starts are indexed in the caller's frame order
+    return W.args.u0 + (F.slot + local) * 256;
+  };
+
+  const long long stride = (long long)gridDim.x * kNetWaves;
+  long long t = (long long)blockIdx.x * kNetWaves + wave;
+  float d[4], gm[4];
+  float *u0 = nullptr;
+  if (t < total) u0 = load(t, d, gm);
+  stage_forward(packs, P, pk, bl);
+  in_pad_border(grid, lane);
+  for (; t < total; t += stride) {
     float sigma;
-    tile_inputs(d, gm, io, lane, sigma);
+    tile_inputs(d, gm, grid, lane, sigma);
 #pragma unroll
     for (int r = 0; r < 4; r++) dkeep[r * 64 + lane] = d[r];
-    const f4 y = net_body(io, pk, bl, lane, nullptr, 0, 0);
-    // starts are indexed in the caller's frame order
-    float *const w = u0 + (F.slot + local) * 256;
+    float *const w = u0;
+    const f4 y = net_body(grid, dbuf, pk, bl, lane, nullptr, 0, 0, [&] {
+      if (t + stride < total) u0 = load(t + stride, d, gm);
+    });
 #pragma unroll
     for (int r = 0; r < 4; r++)
       w[(4 * grp + r) * 16 + col] = dkeep[r * 64 + lane] + sigma * y[r];
