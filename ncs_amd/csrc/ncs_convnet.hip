@@ -183,12 +183,21 @@ __device__ __forceinline__ i2v relu_masked(f4 v, i2v act) {
 }
 
 // A register row written as row y of a [256][32] BF16 buffer in the
-// standard channel order (the activations kept for the backward pass).
+// standard channel order (the activations kept for the backward pass).  Lane
+// (g, x) holds channels 4g.. and 16 + 4g.. of pixel x; exchanged with the
+// lane group next to it (the row swap trades the second half of an even group
+// for the first half of the odd one), every lane has eight channels in a row,
+// 16 (g & 1) + 8 (g >> 1).., and a wave's store is one stretch of 1 KB
+// (8000 tiles, 393 MB of activations: 108.6 -> 101.4 us, with the next tile's
+// inputs loaded under layer 4; two stores of 8 bytes a lane before).
 __device__ __forceinline__ void store_row_std(__bf16 *dst, int y, int lane, i4 v) {
   const int x = lane & 15, g = lane >> 4;
-  __bf16 *px = dst + (y * 16 + x) * kCh;
-  *reinterpret_cast<int2 *>(px + 4 * g) = make_int2(v.x, v.y);
-  *reinterpret_cast<int2 *>(px + 16 + 4 * g) = make_int2(v.z, v.w);
+  const auto a = __builtin_amdgcn_permlane16_swap((unsigned int)v.x, (unsigned int)v.z, false,
+                                                  false);
+  const auto b = __builtin_amdgcn_permlane16_swap((unsigned int)v.y, (unsigned int)v.w, false,
+                                                  false);
+  __bf16 *const px = dst + (y * 16 + x) * kCh + 16 * (g & 1) + 8 * (g >> 1);
+  *reinterpret_cast<i4 *>(px) = (i4){(int)a[0], (int)b[0], (int)a[1], (int)b[1]};
 }
 
 // Layer 1 (2 -> 32 channels), K = tap * 2 + cin padded to 32.  The inputs sit
@@ -234,10 +243,14 @@ __device__ __forceinline__ void layer32(i4 (&act)[16], const i4 *packs_in, const
   const i4 *packs = packs_in + z0;
   const float *bias = bias_in + z0;
   i4 A[2][9];
+  // in the order of their first use, so that the first products need not wait
+  // for the last of them
+  constexpr int order[9] = {3, 0, 4, 1, 5, 2, 6, 7, 8};
 #pragma unroll
-  for (int b = 0; b < 2; b++)
+  for (int i = 0; i < 9; i++)
 #pragma unroll
-    for (int t = 0; t < 9; t++) A[b][t] = packs[(b * 9 + t) * 64 + lane];
+    for (int b = 0; b < 2; b++)
+      A[b][order[i]] = packs[(b * 9 + order[i]) * 64 + lane];
   const f4 c0 = bias4(bias, 0, lane), c1 = bias4(bias, 1, lane);
   const i4 z = {0, 0, 0, 0};
   i4 C[4], L[4], R[4];  // rows y - 1 .. y + 2: centre, dx = -1, dx = +1
@@ -422,13 +435,24 @@ constexpr int kNetWaves = 4;
 constexpr int kFwdPacks = PK_B4 - PK_L1;
 constexpr int kNetFwdLdsBytes = kFwdPacks * 1024 + 128 * 4 + kNetWaves * kNetWaveFloats * 4;
 
-// Copies the forward packs and the biases [b1 | b2 | b3 | b4] into LDS.
+// Copies the forward packs and the biases [b1 | b2 | b3 | b4] into LDS, all
+// of a thread's loads in flight together (one behind the other they delayed a
+// workgroup's first tile by 1 us).
 __device__ __forceinline__ void stage_forward(const i4 *__restrict__ packs,
                                               const float *__restrict__ P, i4 *pk, float *bl) {
-  for (int i = threadIdx.x; i < kFwdPacks * 64; i += blockDim.x) pk[i] = packs[PK_L1 * 64 + i];
-  for (int i = threadIdx.x; i < 97; i += blockDim.x)
-    bl[i] = i < 32 ? P[OFF_B1 + i]
-                   : (i < 64 ? P[OFF_B2 + i - 32] : (i < 96 ? P[OFF_B3 + i - 64] : P[OFF_B4]));
+  constexpr int kThreads = 64 * kNetWaves, kItems = kFwdPacks * 64;
+  constexpr int kEach = (kItems + kThreads - 1) / kThreads;
+  const int tid = threadIdx.x;
+  i4 v[kEach];
+#pragma unroll
+  for (int k = 0; k < kEach; k++) v[k] = packs[PK_L1 * 64 + min(tid + k * kThreads, kItems - 1)];
+  const int layer = tid >> 5;
+  const int at = (layer == 0 ? OFF_B1 : layer == 1 ? OFF_B2 : OFF_B3) + (tid & 31);
+  const float b = P[tid < 96 ? at : OFF_B4];
+#pragma unroll
+  for (int k = 0; k < kEach; k++)
+    if (tid + k * kThreads < kItems) pk[tid + k * kThreads] = v[k];
+  if (tid < 97) bl[tid] = b;
   __syncthreads();
 }
 
@@ -447,13 +471,26 @@ void net_fwd_kernel(const float *__restrict__ xin, float *__restrict__ yout,
   int *const grid = reinterpret_cast<int *>(bl + 128 + wave * kNetWaveFloats);
   float *const dbuf = reinterpret_cast<float *>(grid + kNetGridInts);
   const int col = lane & 15, grp = lane >> 4;
+  float x0[4], x1[4];
+  auto load = [&](long long t) {
+    const float *const x = xin + t * 512;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      x0[k] = x[lane + 64 * k];
+      x1[k] = x[lane + 64 * k + 256];
+    }
+  };
+  const long long stride = (long long)gridDim.x * kNetWaves;
+  long long t = (long long)blockIdx.x * kNetWaves + wave;
+  if (t < n) load(t);
   stage_forward(packs, P, pk, bl);
   in_pad_border(grid, lane);
-  for (long long t = (long long)blockIdx.x * kNetWaves + wave; t < n;
-       t += (long long)gridDim.x * kNetWaves) {
-    for (int i = lane; i < 256; i += 64)
-      in_pad_put(grid, i >> 4, i & 15, xin[t * 512 + i], xin[t * 512 + 256 + i]);
-    const f4 y = net_body(grid, dbuf, pk, bl, lane, acts, n, t, [] {});
+  for (; t < n; t += stride) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) in_pad_put(grid, 4 * k + grp, col, x0[k], x1[k]);
+    const f4 y = net_body(grid, dbuf, pk, bl, lane, acts, n, t, [&] {
+      if (t + stride < n) load(t + stride);
+    });
 #pragma unroll
     for (int r = 0; r < 4; r++) yout[t * 256 + (4 * grp + r) * 16 + col] = y[r];
     wave_sync();
@@ -525,7 +562,15 @@ void net_warm_kernel(WithFrames<NetWarmArgs> W) {
   if (t < total) u0 = load(t, d, gm);
   stage_forward(packs, P, pk, bl);
   in_pad_border(grid, lane);
+  // The two waves of a SIMD start together and run the same tile in the same
+  // time: both would convert, shift and wait in step, with the matrix cores
+  // idle.  Each is favoured on every other tile, which keeps them apart (two
+  // 2048^2 frames, net and solve: 424 -> 418 us; always the same one: 427).
+  bool favoured = 2 * blockIdx.x >= gridDim.x;
   for (; t < total; t += stride) {
+    if (favoured) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+    favoured = !favoured;
     float sigma;
     tile_inputs(d, gm, grid, lane, sigma);
 #pragma unroll
