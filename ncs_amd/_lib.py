@@ -310,10 +310,10 @@ class Context(object):
         total = 0
         keep = []
         counts = {}  # tiles of each distinct frame size
-        last_gamma = None
+        last_gamma = g = None
         for i in range(n):
             d = numpy.ascontiguousarray(datas[i], dtype=numpy.float32)
-            if gammas[i] is not last_gamma:  # one array for all frames: once
+            if g is None or gammas[i] is not last_gamma:  # one array for all frames: once
                 last_gamma = gammas[i]
                 g = numpy.ascontiguousarray(last_gamma, dtype=numpy.float32)
             o = outs[i]
