@@ -25,6 +25,8 @@ hipError_t launch_adu_levels(const uint16_t *adu, const float *offset, const flo
                              const float *gammas, long long stride, const int *t, float *out,
                              float *gamma, long long n, hipStream_t s);
 hipError_t net_pack(const float *P, void *packs, hipStream_t s);
+hipError_t net_pack_forward(const float *P, void *packs, hipStream_t s);
+hipError_t net_pack_backward(const float *P, void *packs, float *gP, hipStream_t s);
 size_t net_packs_bytes();
 hipError_t net_forward(const float *x, float *y, void *acts, const void *packs, const float *P,
                        long long n, int grid, hipStream_t s);
@@ -1214,13 +1216,11 @@ extern "C" int ncs_hip_net_set_weights(ncs_ctx *ctx, const float *params_f32) {
   return NCS_OK;
 }
 
-// Packs `params` (device) into the context's scratch packs, or returns the
-// context's own packs when params is NULL.
-static int packs_for(ncs_ctx *ctx, const float *params, hipStream_t s, const void **packs,
-                     const float **P) {
+// The packs of `params` (device), in the context's scratch (to be filled by
+// the caller), or the context's own when params is NULL.
+static int packs_for(ncs_ctx *ctx, const float *params, void **packs, const float **P) {
   if (params) {
     HIPCHK(ctx->net_tmp_packs.ensure(net_packs_bytes()));
-    HIPCHK(net_pack(params, ctx->net_tmp_packs.p, s));
     *packs = ctx->net_tmp_packs.p;
     *P = params;
     return NCS_OK;
@@ -1257,10 +1257,11 @@ extern "C" int ncs_hip_net_forward(ncs_ctx *ctx, const float *params, const floa
   if (!ctx || !x || !out || n < 0) return fail(NCS_E_ARG, "bad arguments");
   HIPCHK(set_device(ctx));
   hipStream_t s = (hipStream_t)stream;  // 0 = the default (NULL) stream
-  const void *packs;
+  void *packs;
   const float *P;
-  int rc = packs_for(ctx, params, s, &packs, &P);
+  int rc = packs_for(ctx, params, &packs, &P);
   if (rc) return rc;
+  HIPCHK(net_pack_forward(params, packs, s));
   const int grid = net_forward_grid(n, ctx->cus);
   HIPCHK(net_forward(x, out, acts, packs, P, n, grid, s));
   return NCS_OK;
@@ -1274,10 +1275,11 @@ extern "C" int ncs_hip_net_backward(ncs_ctx *ctx, const float *params, const flo
   if (grad_x) return fail(NCS_E_ARG, "the input gradient is not provided (pass NULL)");
   HIPCHK(set_device(ctx));
   hipStream_t s = (hipStream_t)stream;  // 0 = the default (NULL) stream
-  const void *packs;
+  void *packs;
   const float *P;
-  int rc = packs_for(ctx, params, s, &packs, &P);
+  int rc = packs_for(ctx, params, &packs, &P);
   if (rc) return rc;
+  HIPCHK(net_pack_backward(params, packs, grad_params, s));
   HIPCHK(net_backward(x, acts, grad_out, grad_params, packs, n, ctx->cus, s));
   return NCS_OK;
 }

@@ -65,10 +65,17 @@ __device__ __forceinline__ float w_at(const float *P, int off, int cin_n, int co
   return P[off + (co * cin_n + ci) * 9 + tap];
 }
 
-// Builds the BF16 A-operand packs from the FP32 parameters.
-__global__ void net_pack_kernel(const float *__restrict__ P, __bf16 *__restrict__ packs) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= N_PACKS * 512) return;
+// Builds the BF16 A-operand packs [first, end) from the FP32 parameters: the
+// forward pass takes those before PK_B4, the backward pass the others.  Also
+// clears `sums` (may be NULL), the backward pass's gradient: with a launch of
+// its own for that, and all packs for each pass, the backward call took 24.7 us
+// where it takes 23.3 (128 tiles), 51.0 where it takes 49.3 (1024).
+__global__ void net_pack_kernel(const float *__restrict__ P, __bf16 *__restrict__ packs, int first,
+                                int end, float *__restrict__ sums) {
+  const int item = blockIdx.x * blockDim.x + threadIdx.x;
+  if (sums != nullptr && item < N_PARAMS) sums[item] = 0.0f;
+  const int idx = first * 512 + item;
+  if (idx >= end * 512) return;
   const int pack = idx >> 9, lane = (idx >> 3) & 63, e = idx & 7;
   const int i = lane & 15, g = lane >> 4;
   const int k = 8 * g + e;
@@ -1010,21 +1017,34 @@ void net_bwd_kernel(const float *__restrict__ xin, const __bf16 *__restrict__ ac
   }
 }
 
-__global__ void fill_kernel(float *p, long long n, float v) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x)
-    p[i] = v;
-}
-
 // ---------------------------------------------------------------------------
 // launches
 // ---------------------------------------------------------------------------
 
-hipError_t net_pack(const float *P, void *packs, hipStream_t s) {
-  const int total = N_PACKS * 512;
-  hipLaunchKernelGGL(net_pack_kernel, dim3((total + 255) / 256), dim3(256), 0, s, P,
-                     reinterpret_cast<__bf16 *>(packs));
+// Packs what a pass needs of the parameters (NULL: nothing), and clears the
+// N_PARAMS sums when given.
+static hipError_t pack(const float *P, void *packs, int first, int end, float *sums,
+                       hipStream_t s) {
+  if (P == nullptr) end = first;
+  const int items = std::max((end - first) * 512, sums != nullptr ? N_PARAMS : 0);
+  if (items == 0) return hipSuccess;
+  hipLaunchKernelGGL(net_pack_kernel, dim3((items + 255) / 256), dim3(256), 0, s, P,
+                     reinterpret_cast<__bf16 *>(packs), first, end, sums);
   return hipGetLastError();
+}
+hipError_t net_pack(const float *P, void *packs, hipStream_t s) {
+  return pack(P, packs, 0, N_PACKS, nullptr, s);
+}
+hipError_t net_pack_forward(const float *P, void *packs, hipStream_t s) {
+  return pack(P, packs, 0, PK_B4, nullptr, s);
+}
+hipError_t net_pack_backward(const float *P, void *packs, float *gP, hipStream_t s) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(P), g = reinterpret_cast<uintptr_t>(gP);
+  constexpr uintptr_t bytes = N_PARAMS * sizeof(float);
+  if (P == nullptr || p >= g + bytes || g >= p + bytes) return pack(P, packs, PK_B4, N_PACKS, gP, s);
+  // the gradient takes the parameters' place: read them all first
+  const hipError_t e = pack(P, packs, PK_B4, N_PACKS, nullptr, s);
+  return e == hipSuccess ? pack(nullptr, packs, PK_B4, N_PACKS, gP, s) : e;
 }
 
 size_t net_packs_bytes() { return (size_t)N_PACKS * 512 * 2; }
@@ -1051,10 +1071,10 @@ hipError_t net_forward(const float *x, float *y, void *acts, const void *packs, 
   return hipGetLastError();
 }
 
+// gP: cleared by net_pack_backward.
 hipError_t net_backward(const float *x, const void *acts, const float *gout, float *gP,
                         const void *packs, long long n, int cus, hipStream_t s) {
-  hipLaunchKernelGGL(fill_kernel, dim3(64), dim3(256), 0, s, gP, (long long)N_PARAMS, 0.0f);
-  if (n <= 0) return hipGetLastError();
+  if (n <= 0) return hipSuccess;
   const long long pairs = (n + kBwdTeams - 1) / kBwdTeams;
   const int grid = (int)std::max<long long>(1, std::min<long long>(pairs, cus));
   hipLaunchKernelGGL(net_bwd_kernel, dim3(grid), dim3(kBwdTeams * 256), 0, s, x,

@@ -94,3 +94,32 @@ def test_frames_of_a_batch_equal_each_alone(gpu_ctx):
         frames.append(_frame(d, g, geometry=geo))
     batch = _predict(gpu_ctx, frames)
     assert torch.equal(batch, torch.cat([_predict(gpu_ctx, [f]) for f in frames]))
+
+
+def test_backward_clears_and_packs_for_every_caller(gpu_ctx):
+    """The gradient does not depend on where the parameters are: a buffer of
+    their own, the gradient's own buffer, or the context's weights; without
+    tiles it is zero.  One tile: each sum is of one workgroup, in one order."""
+    import torch
+    host = warmstart.init_params(6, last_scale=1.0)
+    p = torch.from_numpy(host).cuda()
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(6)
+    x = torch.randn((1, 2, 16, 16), generator=gen, device="cuda")
+    gy = torch.randn((1, 16, 16), generator=gen, device="cuda")
+    _, acts = _forward(gpu_ctx, p, x)
+
+    def backward(params, grad, n):
+        _lib.check(gpu_ctx.lib.ncs_hip_net_backward(
+            gpu_ctx.handle, params, x.data_ptr(), acts.data_ptr(), gy.data_ptr(),
+            grad.data_ptr(), None, n, torch.cuda.current_stream().cuda_stream), "backward")
+        torch.cuda.synchronize()
+        return grad
+
+    ref = backward(p.data_ptr(), torch.full_like(p, 7.0), 1)
+    assert float(ref.norm()) > 0.0
+    q = p.clone()
+    assert torch.equal(backward(q.data_ptr(), q, 1), ref)
+    warmstart.set_context_weights(host)
+    assert torch.equal(backward(None, torch.full_like(p, 7.0), 1), ref)
+    assert not bool(backward(p.data_ptr(), torch.full_like(p, 7.0), 0).any())
