@@ -506,7 +506,6 @@ enum LsResult { LS_CONTINUE = 0, LS_ACCEPT = 1, LS_FAIL_PRECISION = -1,
                 LS_FAIL_MINSTEP = -2, LS_FAIL_INCREASE = -3 };
 
 struct MtState {
-  float ll_start, nc_start;  // not the search's: the parts of f(u_start)
   float stx, fx, dx, sty, fy, dy;
   float stmin, stmax, width, prev_width;
   float dginit, dgtest;
@@ -682,10 +681,6 @@ __device__ __forceinline__ int mt_post(MtState &S, float &stp, float f, float dg
 // ---------------------------------------------------------------------------
 // The persistent solver kernel
 // ---------------------------------------------------------------------------
-
-// The reported cost is f(u_start) plus the steps' sum while that sum is at
-// most this share of it.
-constexpr float kCostSum = 0.25f;
 
 // Dynamic ranges a wave takes tiles from: its home range and the next one.
 constexpr int kScan = 2;
@@ -896,7 +891,6 @@ void solve_kernel(WithFrames<SolveArgs> L) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform
   constexpr bool kCacheIv = M <= 3;  // keep 1/(u+gamma) across iterations
   constexpr bool kCorr = M <= kCorrHistory;
-  constexpr bool kSumCost = !F16 && M <= 5;
   MtState &mt_lds = mt_state[wave];
   constexpr bool kReg = M >= kRegPair;
   constexpr int kRing = ring_slots(M);
@@ -1058,7 +1052,6 @@ void solve_kernel(WithFrames<SolveArgs> L) {
     // direction, for the likelihood trial) and one back (the likelihood
     // gradient).  Dot products are basis-independent.
     float gs[4], gncs[4], zs[4], iv[4];  // spectral g, K u; pixel 1/(u+gamma)
-    float f = 0.0f;  // f(u) - f(u_start): only differences drive the search
     // Basis changes run on the FP16 matrix cores (22-bit operands) until the
     // gradient is within kF16Floor of the stop rule's scale, and in FP32
     // after that: a default-tolerance solve (eps 1e-5) stops before the
@@ -1071,13 +1064,6 @@ void solve_kernel(WithFrames<SolveArgs> L) {
       const bool warm = A.u0 != nullptr || A.lin_start;
       if (!warm) {
         ll_grad_lane(u, gm, c, lin, gll, iv);
-        if (kSumCost && A.cost != nullptr) {
-          float red[2] = {ll_value_lane(u, gm, c, lin),
-                          zs[0] * gncs[0] + zs[1] * gncs[1] + (zs[2] * gncs[2] + zs[3] * gncs[3])};
-          wave_sum<2>(red);
-          mt_lds.ll_start = red[0];
-          mt_lds.nc_start = 0.5f * alpha * red[1];
-        }
       } else {
         // warm start: keep it unless the plain start scores a lower cost
         float both[4];
@@ -1140,12 +1126,7 @@ void solve_kernel(WithFrames<SolveArgs> L) {
         wave_sum<4>(both);
         const float f_plain = both[0] + 0.5f * alpha * both[1];
         const float f_warm = both[2] + 0.5f * alpha * both[3];
-        const bool keep = !A.fallback || f_warm < f_plain || !(f_plain == f_plain);
-        if (kSumCost) {
-          mt_lds.ll_start = keep ? both[2] : both[0];
-          mt_lds.nc_start = 0.5f * alpha * (keep ? both[3] : both[1]);
-        }
-        if (keep) {
+        if (!A.fallback || f_warm < f_plain || !(f_plain == f_plain)) {
 #pragma unroll
           for (int r = 0; r < 4; r++) {
             u[r] = w[r];
@@ -1278,7 +1259,7 @@ void solve_kernel(WithFrames<SolveArgs> L) {
               asm volatile("" ::: "memory");
               ll_trial<PAD, kCacheIv>(tstep, u, dp, gm, c, lin, iv, gt, ivt, red);
               asm volatile("" ::: "memory");
-                    phi = red[0] + alpha * tstep * (a1 + 0.5f * tstep * a2);
+              phi = red[0] + alpha * tstep * (a1 + 0.5f * tstep * a2);
               const float dpt = red[1] + alpha * (a1 + tstep * a2);
               ls = mt_post(S_, tstep, phi, dpt, A);
               dphi_acc = dpt;
@@ -1298,7 +1279,7 @@ void solve_kernel(WithFrames<SolveArgs> L) {
             if (!(tstep >= A.min_step)) { ls = LS_FAIL_MINSTEP; break; }
             if (trials >= A.max_ls) { ls = LS_FAIL_PRECISION; break; }
             ll_trial<PAD, kCacheIv>(tstep, u, dp, gm, c, lin, iv, gt, ivt, red);
-                trials++;
+            trials++;
             phi = red[0] + alpha * tstep * (a1 + 0.5f * tstep * a2);
           }
         }
@@ -1320,8 +1301,6 @@ void solve_kernel(WithFrames<SolveArgs> L) {
         if (restart) {
           float nw[4] = {0.f, 0.f, 0.f, 0.f}, ng[4];
           load_tile(F, G, t, u, ng, nw);
-          f = 0.0f;
-          if (kSumCost) mt_lds.ll_start = __builtin_nanf("");  // not kept for it
         }
         corr_h0 = false;
         exact = true;
@@ -1393,9 +1372,6 @@ void solve_kernel(WithFrames<SolveArgs> L) {
         n_inc = 0;
       }
       to_spec16(gt, T, GB, 1.0f, gts, exact);
-      if (kSumCost) {  // phi is uniform: a scalar register, where none of 96 is free
-        f = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(f + phi)));
-      }
       // y.s = t (phi'(t) - phi'(0)) needs no reduction; the third slot is
       // y.y for the scalar initial Hessian, the mean curvature for the
       // spectral one
@@ -1548,30 +1524,19 @@ void solve_kernel(WithFrames<SolveArgs> L) {
       load_tile(frames[fn], Gn, tn, nd, ng, nw);
     }
 
-    // The cost at the returned point (when asked for): the start's plus the
-    // steps', which the search formed to FP32 accuracy.  Evaluated afresh, NC
-    // from an exact transform of u, only where that sum is not small beside
-    // the cost (a far start's cost would carry the start's rounding), where
-    // the start's overflowed, after a restart, and in the builds that have no
-    // register for it (kSumCost; the FP16 split spilled 7 more and lost 6%).
-    // An evaluation for each tile took 268 us where this takes 255 (4 x 2048^2,
-    // linear start, history 1; 253.5 with no cost asked for), and 394 where
-    // this takes 385 from the plain start at history 5.  Against 64 bits both
-    // are off by 6.6e-8 to 6.9e-8 in the 2-norm.
+    // final cost at the returned point (when asked for), NC from an exact
+    // transform of u.  It costs about 5% of a linear-start tile, but the start's
+    // cost plus the steps', which need no evaluation, was further from 64 bits
+    // (6.7e-8 to 6.9e-8 in the 2-norm, 6.6e-8 to 6.7e-8 so).
+    float f = 0.0f;
     if (A.cost != nullptr) {
-      const float fu = mt_lds.ll_start + (mt_lds.nc_start + f);
-      if (kSumCost && fabsf(f) <= kCostSum * fabsf(fu) && fabsf(fu) < INFINITY) {
-        f = fu;
-      } else {
-        if (kSumCost) asm volatile("" : "+v"(u[0]));  // not ahead of the branch
-        to_spec16<false>(u, T, GB, st, zs, exact);
-        nc_spec<GEN>(zs, T, gncs);
-        float red[2];
-        red[0] = ll_value_lane(u, gm, c, lin);
-        red[1] = zs[0] * gncs[0] + zs[1] * gncs[1] + (zs[2] * gncs[2] + zs[3] * gncs[3]);
-        wave_sum<2>(red);
-        f = red[0] + 0.5f * alpha * red[1];
-      }
+      to_spec16<false>(u, T, GB, st, zs, exact);
+      nc_spec<GEN>(zs, T, gncs);
+      float red[2];
+      red[0] = ll_value_lane(u, gm, c, lin);
+      red[1] = zs[0] * gncs[0] + zs[1] * gncs[1] + (zs[2] * gncs[2] + zs[3] * gncs[3]);
+      wave_sum<2>(red);
+      f = red[0] + 0.5f * alpha * red[1];
     }
 
     // stitch the owned interior and per-tile results (per-tile arrays in the
