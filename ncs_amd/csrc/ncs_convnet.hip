@@ -699,8 +699,9 @@ __device__ __forceinline__ void grad_w32(const LdsByte *dz, const int (&oz)[2],
 // rows, masked by the ReLU of the activations there, as BF16 in registers:
 // the convolution of dz with the flipped, transposed weights (packs: the
 // lane's entries of the nine taps, read from L2 at each use: kept in
-// registers over the tiles they spilled), each accumulator from zero.  z points at the lane's pixel of padded
-// row 8 h, act at the lane's four channels of row 8 h's pixels (padded).
+// registers over the tiles they spilled), each accumulator from zero.  z points
+// at the lane's pixel of padded row 8 h, act at the lane's four channels of
+// row 8 h's pixels (padded).
 __device__ __forceinline__ void grad_data32(const LdsByte *z, const LdsByte *act,
                                             const i4 *__restrict__ packs, i2v (&out)[8]) {
   i4 A[9];
@@ -759,6 +760,34 @@ __device__ __forceinline__ void put_planes(LdsByte *planes, int row, int col, sh
       *reinterpret_cast<__attribute__((address_space(3))) short *>(
           planes + dx * kPlaneBytes + (row + 1) * 32 + 2 * x) = v;
   }
+}
+
+// Layer 4's weight gradient (input channel ci, tap tp) over a workgroup's tiles
+// first + k step + (0 .. kBwdTeams - 1) in plain FP32, in-tile taps only.  It
+// takes the place of the splits' matrix products where those do not hold: a
+// sum that is not finite (dL/dout past BF16's largest value splits into an
+// infinity, and a remainder's or a border's zero times an infinite activation
+// is NaN), or one so small that dL/dout's remainders may have been below
+// BF16's smallest value, 2^-133.  Rare, and slow: one thread per sum.
+constexpr float kW4Small = 0x1p-96f;
+__device__ float w4_fp32(const __bf16 *a3, const float *gout, int ci, int tp, long long first,
+                         long long step, long long n) {
+  const int dy = tp / 3 - 1, dx = tp % 3 - 1;
+  float sum = 0.0f;
+#pragma unroll 1
+  for (long long t0 = first; t0 < n; t0 += step)
+#pragma unroll 1
+    for (long long t = t0; t < n && t < t0 + kBwdTeams; t++) {
+      float s = 0.0f;
+#pragma unroll 1
+      for (int p = 0; p < 256; p++) {
+        const int y = (p >> 4) + dy, x = (p & 15) + dx;
+        if (y >= 0 && y < 16 && x >= 0 && x < 16)
+          s += gout[t * 256 + p] * (float)a3[(t * 256 + y * 16 + x) * kCh + ci];
+      }
+      sum += s;
+    }
+  return sum;
 }
 
 __global__ __launch_bounds__(kBwdTeams * 256) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -830,8 +859,9 @@ void net_bwd_kernel(const float *__restrict__ xin, const __bf16 *__restrict__ ac
     for (int y = 0; y < 8; y++)
       *reinterpret_cast<__attribute__((address_space(3))) i2v *>(dst + own0 + y * kRowBytes) = v[y];
   };
-  // dL/dout of the tile as three BF16 splits (their sum is the FP32 value;
-  // a value past BF16's range keeps its first split only)
+  // dL/dout of the tile as three BF16 splits, whose sum is the FP32 value
+  // (but for values past BF16's largest and remainders below its smallest,
+  // see w4_fp32)
   auto put_dy = [&](float v) {
     db4 += v;
     const int row = tid >> 4, col = tid & 15;
@@ -1007,6 +1037,8 @@ void net_bwd_kernel(const float *__restrict__ xin, const __bf16 *__restrict__ ac
     float v = 0.0f;
 #pragma unroll
     for (int m = 0; m < kBwdTeams * 3; m++) v += sum4[(m * 9 + tp) * kCh + ci];
+    if (!(fabsf(v) < INFINITY) || (v != 0.0f && fabsf(v) < kW4Small))
+      v = w4_fp32(acts + 2 * n * 256 * kCh, gout, ci, tp, first, step, n);
     atomicAdd(&gP[OFF_W4 + threadIdx.x], v);
   }
   if (threadIdx.x == OFF_B4 - OFF_W4) {
