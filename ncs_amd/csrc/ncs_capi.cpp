@@ -120,14 +120,14 @@ struct Schedule {
 // Key of an autotuned schedule: mask kind, padded geometry, precision.
 typedef std::array<bool, 3> TuneKey;
 
-// The last pipeline replay that took its turn on the PCIe link (see
-// takes_turns): what it does, and the events behind its transfers.  The
-// pipelines of a context share it, each from its own thread if need be.
+// The last replay whose download took its turn on the PCIe link (see
+// takes_turns): its pipeline and the event behind it.  The pipelines of a
+// context share it, each from its own thread if need be; a pipeline takes
+// itself out before its events go.
 struct ReplayLine {
   std::mutex mu;
-  std::shared_ptr<const std::string> work;  // null: no such replay
-  hipEvent_t up = nullptr, down = nullptr;
-  bool like(const std::shared_ptr<const std::string> &w) const { return work && *work == *w; }
+  const ncs_pipeline *owner = nullptr;
+  hipEvent_t done = nullptr;
 };
 
 struct ncs_ctx {
@@ -292,8 +292,7 @@ extern "C" int ncs_hip_create(int device, ncs_ctx **out) {
   std::snprintf(c->arch, sizeof(c->arch), "%s", prop.gcnArchName);
   HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   HIPCHK(hipEventCreateWithFlags(&c->frames_event, hipEventDisableTiming));
-  for (hipEvent_t *ev : {&c->solve_done, &c->line.up, &c->line.down})
-    HIPCHK(hipEventCreateWithFlags(ev, hipEventDisableTiming));
+  HIPCHK(hipEventCreateWithFlags(&c->solve_done, hipEventDisableTiming));
   HIPCHK(c->queue.ensure(3 * kQueueBytes));
   const int rc = scratch_on_device(device, &c->scratch);
   if (rc) return rc;
@@ -309,8 +308,7 @@ extern "C" void ncs_hip_destroy(ncs_ctx *ctx) {
                     &ctx->net_params, &ctx->net_packs, &ctx->net_tmp_packs, &ctx->u0_buf};
   for (DevBuf *b : bufs) b->release();
   if (ctx->frames_event) (void)hipEventDestroy(ctx->frames_event);
-  for (hipEvent_t ev : {ctx->solve_done, ctx->line.up, ctx->line.down})
-    if (ev) (void)hipEventDestroy(ev);
+  if (ctx->solve_done) (void)hipEventDestroy(ctx->solve_done);
   if (ctx->frames_staging) (void)hipHostFree(ctx->frames_staging);
   if (ctx->stage) (void)hipHostFree(ctx->stage);
   for (hipEvent_t e : ctx->stage_event)
@@ -1489,7 +1487,7 @@ struct ncs_pipeline {
   std::vector<size_t> off;      // first pixel of each frame in the packed buffers
   size_t pix = 0;
   long long total = 0;
-  std::shared_ptr<const std::string> work;  // frames, input and parameters
+  std::string work;  // frames, input and parameters
   bool pad = false, general = false, keep = false, learned = false;
   int win = 16;  // the context's window side when the pipeline was created
   Schedule sched;
@@ -1513,7 +1511,11 @@ struct ncs_pipeline {
 
 extern "C" void ncs_hip_pipeline_destroy(ncs_pipeline *pl) {
   if (!pl) return;
-  if (pl->ctx) (void)hipSetDevice(pl->ctx->device);
+  if (pl->ctx) {
+    (void)hipSetDevice(pl->ctx->device);
+    std::lock_guard<std::mutex> lk(pl->ctx->line.mu);
+    if (pl->ctx->line.owner == pl) pl->ctx->line.owner = nullptr;
+  }
   if (pl->launched > pl->waited)
     (void)hipEventSynchronize(pl->done[(pl->launched - 1) % kReplaySlots]);
   if (pl->exec) (void)hipGraphExecDestroy(pl->exec);
@@ -1616,9 +1618,9 @@ extern "C" int ncs_hip_pipeline_create(ncs_ctx *ctx, const ncs_pipeline_frame *f
   for (int k = 0; k < kReplaySlots; k++)
     HIPCHK(hipEventCreateWithFlags(&pl->done[k], hipEventDisableTiming));
   pl->gamma_set.assign(n_frames, 0);
-  std::string work(reinterpret_cast<const char *>(frames), n_frames * sizeof *frames);
-  work.append(reinterpret_cast<const char *>(params), sizeof *params).push_back((char)input_format);
-  pl->work = std::make_shared<const std::string>(std::move(work));
+  pl->work.assign(reinterpret_cast<const char *>(frames), n_frames * sizeof *frames);
+  pl->work.append(reinterpret_cast<const char *>(params), sizeof *params);
+  pl->work.push_back((char)input_format);
   pl->levels.assign(n_frames, 1);
   pl->level_points.resize(n_frames);
   pl->sched = resolve_schedule(ctx, params, pl->pad, pl->total);
@@ -1802,63 +1804,52 @@ static int build_pipeline_graph(ncs_pipeline *pl) {
   return NCS_OK;
 }
 
-// Replays of like pipelines take turns on the PCIe link: the uploads of one
-// wait for those of the one enqueued before it, and so do the downloads.
-// Left alone, two of them share the link each way: neither has its image
-// before both are nearly through, and the link then idles for the next upload
-// and solve.  Four 2304 x 2304 frames through two pipelines went from 2295 to
-// 2032 us, the first image from 1140 to 780.
+// Downloads of like pipelines take turns on the PCIe link: a replay's waits
+// for that of the other pipeline's replay before it.  Left alone, two of them
+// share the link: neither has its image before both are nearly through, and
+// the link then idles for the next upload and solve.  Six 2304 x 2304 frames
+// through two pipelines take 3031 us instead of 3285 (16-bit input) and 3719
+// instead of 4429 (FP32).
 // Only where the wait pays and cannot cost:
 //  * both run on their pipelines' own streams with no replay before them that
 //    the caller has not waited for, so what is waited for is under way;
 //  * both do the same work, so the one enqueued first is ready first;
-//  * the images are large: the four event operations cost the link some 30 us
-//    a replay.  Unordered and ordered, us for 2 and for 6 frames: 724 x 724
-//    165, 440 and 195, 496; 1024 x 1024 287, 777 and 304, 749; 1448 x 1448
-//    532, 1379 and 519, 1257.
+//  * the images are large: the wait costs the link some 10 us a replay.
+// Uploads do not take turns.  That gained more (2894 and 3417 us), but HIP
+// deals a process's streams out to four hardware queues, and where the two
+// pipelines' share one the wait ahead of an upload stood behind the other's
+// solve, so that nothing overlapped: 4640 and 5650 us.  There the downloads'
+// turns make 3814 us of 3741 and 4234 of 4162.
 constexpr size_t kTurnBytes = 8 << 20;
 
 static bool takes_turns(const ncs_pipeline *pl, hipStream_t stream) {
   return !stream && pl->launched == pl->waited && pl->pix * sizeof(float) >= kTurnBytes;
 }
 
-// Enqueues one replay on s: upload of every frame, the graph, download of
-// every frame and of the per-tile results into the replay's slot.  The lock
-// is not held over the copies, which block where the memory is pageable: a
-// replay that another thread overtakes there goes unordered.
-static hipError_t enqueue_replay(ncs_pipeline *pl, hipStream_t s, int slot, bool in_turn) {
+// Makes s wait for the replay in the line, if another, like pipeline's.
+static hipError_t await_turn(const ncs_pipeline *pl, hipStream_t s) {
   ReplayLine &line = pl->ctx->line;
-  bool after = false;
-  hipError_t e = hipSuccess;
-  if (in_turn) {
-    std::lock_guard<std::mutex> lk(line.mu);
-    after = line.like(pl->work);
-    if (after) e = hipStreamWaitEvent(s, line.up, 0);
-  }
+  std::lock_guard<std::mutex> lk(line.mu);
+  if (!line.owner || line.owner == pl || line.owner->work != pl->work) return hipSuccess;
+  return hipStreamWaitEvent(s, line.done, 0);
+}
+
+// Enqueues one replay on s: upload of every frame, the graph, download of
+// every frame and of the per-tile results into the replay's slot.
+static hipError_t enqueue_replay(ncs_pipeline *pl, hipStream_t s, int slot, bool in_turn) {
   char *dev_in = pl->input == NCS_INPUT_ADU_U16 ? pl->raw.as<char>() : pl->data.as<char>();
+  hipError_t e = hipSuccess;
   for (int i = 0; i < pl->n && e == hipSuccess; i++)
     e = hipMemcpyAsync(dev_in + pl->off[i] * pl->elem, pl->cur_in[i],
                        frame_pixels(pl->shape[i]) * pl->elem, hipMemcpyHostToDevice, s);
-  if (in_turn && e == hipSuccess) {
-    std::lock_guard<std::mutex> lk(line.mu);
-    e = hipEventRecord(line.up, s);
-  }
   if (e == hipSuccess) e = hipGraphLaunch(pl->exec, s);
-  if (after && e == hipSuccess) {
-    std::lock_guard<std::mutex> lk(line.mu);
-    if (line.like(pl->work)) e = hipStreamWaitEvent(s, line.down, 0);
-  }
+  if (e == hipSuccess && in_turn) e = await_turn(pl, s);
   for (int i = 0; i < pl->n && e == hipSuccess; i++)
     e = hipMemcpyAsync(pl->cur_out[i], pl->out.as<float>() + pl->off[i],
                        frame_pixels(pl->shape[i]) * sizeof(float), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess && pl->keep) {
     e = hipMemcpyAsync(pl->h_res[slot], pl->results.p, (size_t)pl->total * 12,
                        hipMemcpyDeviceToHost, s);
-  }
-  if (in_turn && e == hipSuccess) {
-    std::lock_guard<std::mutex> lk(line.mu);
-    e = hipEventRecord(line.down, s);
-    line.work = e == hipSuccess ? pl->work : nullptr;
   }
   return e;
 }
@@ -1905,12 +1896,18 @@ extern "C" int ncs_hip_pipeline_launch(ncs_pipeline *pl, const void *const *inpu
   // stream waits on the device for the previous one
   if (seq > pl->waited && s != pl->last_stream)
     e = hipStreamWaitEvent(s, pl->done[(seq - 1) % kReplaySlots], 0);
-  if (e == hipSuccess) e = enqueue_replay(pl, s, slot, takes_turns(pl, (hipStream_t)stream));
+  const bool in_turn = takes_turns(pl, (hipStream_t)stream);
+  if (e == hipSuccess) e = enqueue_replay(pl, s, slot, in_turn);
   // whatever was enqueued is covered by the replay's event
   hipError_t e2 = hipEventRecord(pl->done[slot], s);
   if (e2 == hipSuccess) {
     pl->launched = seq + 1;
     pl->last_stream = s;
+    if (in_turn && e == hipSuccess) {
+      std::lock_guard<std::mutex> lk(ctx->line.mu);
+      ctx->line.owner = pl;
+      ctx->line.done = pl->done[slot];
+    }
   }
   HIPCHK(e);
   HIPCHK(e2);
