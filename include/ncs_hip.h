@@ -173,7 +173,12 @@ int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int n_frames,
  * context share its frame table and work queue: one enqueued on another
  * stream than the context's previous solve waits on the device for that
  * solve to complete, so calls on several streams are safe but run one after
- * the other (use one context per stream for concurrent solves). */
+ * the other (use one context per stream for concurrent solves).  Captured into
+ * a graph, solves are ordered within their capture only: replays may run beside
+ * the context's other solves, but not beside each other; those of more than 32
+ * frames or with the learned start use the context's frame table and start
+ * buffer, so nothing else may.  Such captures are refused (NCS_E_HIP) once the
+ * context has solved on another stream. */
 int ncs_hip_reduce_frames_device(ncs_ctx *ctx, const ncs_frame *frames,
                                  int n_frames, const ncs_params *params,
                                  const float *u0_tiles, int *iterations,

@@ -176,6 +176,10 @@ struct ncs_ctx {
   hipEvent_t solve_done = nullptr;
   hipStream_t solve_stream = nullptr;
   bool solve_pending = false;
+  // the same for solves captured into a graph, within one capture
+  hipEvent_t captured_done = nullptr;
+  hipStream_t captured_stream = nullptr;
+  unsigned long long captured_id = 0;
   // device address of the allocation-free entry point's scratch on this GPU
   void *scratch = nullptr;
   // pinned staging of the host-memory entry points: kStageSlots slots, each
@@ -185,22 +189,53 @@ struct ncs_ctx {
   ReplayLine line;
 };
 
-// Orders a solve on stream s after the context's previous one.
-static hipError_t order_after_previous(ncs_ctx *ctx, hipStream_t s) {
+// Whether a stream is being captured, and the capture's number.
+struct Capture {
+  bool on = false;
+  unsigned long long id = 0;
+};
+
+static Capture capture_of(hipStream_t s) {
+  Capture c;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamGetCaptureInfo(s, &st, &c.id) != hipSuccess) {
+    (void)hipGetLastError();
+    st = hipStreamCaptureStatusActive;
+    c.id = 0;
+  }
+  c.on = st != hipStreamCaptureStatusNone;
+  return c;
+}
+
+// Orders a solve on stream s after the context's previous one.  An event
+// links streams only within one capture or outside of any, so captured solves
+// are ordered among those of their capture, and the others among themselves:
+// with one event for all, a capture after a solve on another stream was
+// refused, and a solve after a capture waited for an event that no stream
+// had recorded.
+static hipError_t order_after_previous(ncs_ctx *ctx, hipStream_t s, const Capture &cap) {
+  if (cap.on) {
+    if (cap.id != 0 && ctx->captured_id == cap.id && ctx->captured_stream != s)
+      return hipStreamWaitEvent(s, ctx->captured_done, 0);
+    return hipSuccess;
+  }
   if (ctx->solve_pending && ctx->solve_stream != s)
     return hipStreamWaitEvent(s, ctx->solve_done, 0);
   return hipSuccess;
 }
 
-static hipError_t mark_solve(ncs_ctx *ctx, hipStream_t s) {
-  hipError_t e = hipEventRecord(ctx->solve_done, s);
-  if (e == hipSuccess) {
+static hipError_t mark_solve(ncs_ctx *ctx, hipStream_t s, const Capture &cap) {
+  hipError_t e = hipEventRecord(cap.on ? ctx->captured_done : ctx->solve_done, s);
+  if (e != hipSuccess) return e;
+  if (cap.on) {
+    ctx->captured_stream = s;
+    ctx->captured_id = cap.id;
+  } else {
     ctx->solve_stream = s;
     ctx->solve_pending = true;
   }
-  return e;
+  return hipSuccess;
 }
-
 
 static hipError_t set_device(ncs_ctx *ctx) { return hipSetDevice(ctx->device); }
 
@@ -292,7 +327,8 @@ extern "C" int ncs_hip_create(int device, ncs_ctx **out) {
   std::snprintf(c->arch, sizeof(c->arch), "%s", prop.gcnArchName);
   HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   HIPCHK(hipEventCreateWithFlags(&c->frames_event, hipEventDisableTiming));
-  HIPCHK(hipEventCreateWithFlags(&c->solve_done, hipEventDisableTiming));
+  for (hipEvent_t *ev : {&c->solve_done, &c->captured_done})
+    HIPCHK(hipEventCreateWithFlags(ev, hipEventDisableTiming));
   HIPCHK(c->queue.ensure(3 * kQueueBytes));
   const int rc = scratch_on_device(device, &c->scratch);
   if (rc) return rc;
@@ -308,7 +344,8 @@ extern "C" void ncs_hip_destroy(ncs_ctx *ctx) {
                     &ctx->net_params, &ctx->net_packs, &ctx->net_tmp_packs, &ctx->u0_buf};
   for (DevBuf *b : bufs) b->release();
   if (ctx->frames_event) (void)hipEventDestroy(ctx->frames_event);
-  if (ctx->solve_done) (void)hipEventDestroy(ctx->solve_done);
+  for (hipEvent_t ev : {ctx->solve_done, ctx->captured_done})
+    if (ev) (void)hipEventDestroy(ev);
   if (ctx->frames_staging) (void)hipHostFree(ctx->frames_staging);
   if (ctx->stage) (void)hipHostFree(ctx->stage);
   for (hipEvent_t e : ctx->stage_event)
@@ -779,11 +816,11 @@ static hipError_t launch_schedule(const ncs_ctx *ctx, const Schedule &sc, bool p
 // instead of 253.5, with the default parameters 376 instead of 379.  A set
 // that is not known to be clear (the first, and after a failed launch) is
 // reset; so is the third one, for captured solves, whose replays the context
-// does not see.
+// does not see (they may run beside its other solves, not beside each other).
 static int enqueue_solve(ncs_ctx *ctx, const FrameDev *d_frames, const FrameDev *inline_frames,
                          int n_frames, bool pad, long long total, const ncs_params *p,
                          const float *u0, int *iters, int *status, float *cost,
-                         unsigned int *queue, hipStream_t s) {
+                         unsigned int *queue, hipStream_t s, const Capture &cap = Capture()) {
   if (!ctx->has_mask) return fail(NCS_E_NOMASK, "no OTF mask set");
   if (total <= 0) return NCS_OK;
   const Schedule sc = resolve_schedule(ctx, p, pad, total);
@@ -793,12 +830,7 @@ static int enqueue_solve(ncs_ctx *ctx, const FrameDev *d_frames, const FrameDev 
     HIPCHK(launch_schedule(ctx, sc, pad, total, s, a, inline_frames));
     return NCS_OK;
   }
-  hipStreamCaptureStatus cap;
-  if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-    (void)hipGetLastError();
-    cap = hipStreamCaptureStatusActive;
-  }
-  if (cap != hipStreamCaptureStatusNone) {
+  if (cap.on) {
     a.queue = ctx->counters(2);
     HIPCHK(launch_schedule(ctx, sc, pad, total, s, a, inline_frames));
     return NCS_OK;
@@ -837,7 +869,13 @@ extern "C" int ncs_hip_reduce_frames_device(ncs_ctx *ctx, const ncs_frame *frame
   if (rc) return rc;
   HIPCHK(set_device(ctx));
   hipStream_t s = (hipStream_t)stream;  // 0 = the default (NULL) stream
-  HIPCHK(order_after_previous(ctx, s));
+  const Capture cap = capture_of(s);
+  // such a solve's replays read what the context's buffers hold by then
+  if (cap.on && ctx->solve_pending && ctx->solve_stream != s &&
+      (n_frames > kInlineFrames || params->start == NCS_START_LEARNED))
+    return fail(NCS_E_HIP, "a context in use elsewhere captures up to " +
+                               std::to_string(kInlineFrames) + " frames, without a learned start");
+  HIPCHK(order_after_previous(ctx, s, cap));
   schedule_small_first(fd, total);
   const FrameDev *table = nullptr;
   rc = upload_frames(ctx, fd, s, &table);
@@ -851,9 +889,9 @@ extern "C" int ncs_hip_reduce_frames_device(ncs_ctx *ctx, const ncs_frame *frame
     u0 = ctx->u0_buf.as<float>();
   }
   rc = enqueue_solve(ctx, table, fd.data(), n_frames, any_pad(ctx, frames, n_frames), total,
-                     params, u0, iterations, status, cost, nullptr, s);
+                     params, u0, iterations, status, cost, nullptr, s, cap);
   if (rc) return rc;
-  HIPCHK(mark_solve(ctx, s));
+  HIPCHK(mark_solve(ctx, s, cap));
   return NCS_OK;
 }
 
@@ -1069,7 +1107,7 @@ extern "C" int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int 
   if (rc) return rc;
   HIPCHK(set_device(ctx));
   hipStream_t s = ctx->stream;
-  HIPCHK(order_after_previous(ctx, s));
+  HIPCHK(order_after_previous(ctx, s, Capture()));
   // Device layout, one linear region each way: in = every frame's data, then
   // the distinct gammas, packed [H][W]; out = every frame's image, then the
   // per-tile results that are asked for.
@@ -1136,7 +1174,7 @@ extern "C" int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int 
                          status ? reinterpret_cast<int *>(d_out + r_off[1]) : nullptr,
                          cost ? reinterpret_cast<float *>(d_out + r_off[2]) : nullptr, nullptr, s);
     if (rc == NCS_OK && !direct) e = download_rows(ctx, out, d_out, out_bytes, s);
-    if (rc == NCS_OK && e == hipSuccess) e = mark_solve(ctx, s);
+    if (rc == NCS_OK && e == hipSuccess) e = mark_solve(ctx, s, Capture());
   }
   // whatever was enqueued is complete before the caller's memory is let go
   const hipError_t e2 = hipStreamSynchronize(s);
