@@ -733,12 +733,17 @@ static int default_group(const ncs_ctx *ctx, long long total) {
   return total <= 4LL * ctx->cus ? 1 : 4;
 }
 
-// Waves of a schedule's kernel one CU holds at once (asked once per kernel).
+// Waves of a schedule's kernel one CU holds at once; 0 where no workgroup fits
+// or the query fails, which is not kept: a failed query would otherwise hold
+// the kernel to the fallback for the context's life.
 static int occupancy(const ncs_ctx *ctx, int history, bool pad, bool f16, int wpg) {
   int &w = ctx->waves_per_cu[history][ctx->general][pad][f16][wpg];
-  if (w == 0) w = std::max(1, solve_waves_per_cu(history, ctx->general, pad, f16, wpg));
+  if (w == 0) w = std::max(0, solve_waves_per_cu(history, ctx->general, pad, f16, wpg));
   return w;
 }
+
+// The grid of a kernel whose occupancy is not known.
+constexpr int kWavesUnknown = 8;
 
 // The schedule of a solve of `total` tiles: explicit params win, then the
 // autotuned schedule of this mask kind and geometry, then history 5,
@@ -754,10 +759,14 @@ static Schedule resolve_schedule(const ncs_ctx *ctx, const ncs_params *p, bool p
   s.f16 = f16;
   s.history = p->history > 0 ? p->history : d.history;
   s.wpg = p->waves_per_group > 0 ? p->waves_per_group : d.wpg;
+  // (a group nobody asked for gives way where it does not fit)
+  if (p->waves_per_group <= 0 && s.wpg > 1 && occupancy(ctx, s.history, pad, s.f16, s.wpg) == 0)
+    s.wpg = 1;
   // a tuned grid only applies to the depth and workgroup size it was tuned for
   const bool same = s.history == d.history && s.wpg == d.wpg;
   s.waves_per_cu = p->waves_per_cu > 0 ? p->waves_per_cu : (same ? d.waves_per_cu : 0);
   if (s.waves_per_cu <= 0) s.waves_per_cu = occupancy(ctx, s.history, pad, s.f16, s.wpg);
+  if (s.waves_per_cu <= 0) s.waves_per_cu = kWavesUnknown;
   return s;
 }
 
@@ -1435,7 +1444,9 @@ extern "C" int ncs_hip_autotune(ncs_ctx *ctx, const ncs_frame *frames, int n_fra
   def.history = base->history > 0 ? base->history : 5;
   def.wpg = default_group(ctx, total);
   def.f16 = f16;
+  if (occupancy(ctx, def.history, pad, f16, def.wpg) == 0) def.wpg = 1;
   def.waves_per_cu = occupancy(ctx, def.history, pad, f16, def.wpg);
+  if (def.waves_per_cu == 0) def.waves_per_cu = kWavesUnknown;
   float ms_def = 0.0f;
   e = time_one(def, &ms_def);
   struct Cand {
@@ -1453,6 +1464,7 @@ extern "C" int ncs_hip_autotune(ncs_ctx *ctx, const ncs_frame *frames, int n_fra
     for (int wpg : groups) {
       if (e != hipSuccess) break;
       const int occ = occupancy(ctx, m, pad, f16, wpg);
+      if (occ == 0) continue;
       std::vector<int> grid = {occ, std::max(wpg, (occ * 3 / 4) / wpg * wpg),
                                std::max(wpg, (occ / 2) / wpg * wpg)};
       std::sort(grid.begin(), grid.end());

@@ -1686,8 +1686,10 @@ int solve_waves_per_cu(int m, bool general, bool pad, bool f16, int wpg) {
   int blocks = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
           &blocks, reinterpret_cast<const void *>(fn), kWave * wpg, solve_lds_bytes(m, wpg)) !=
-      hipSuccess)
+      hipSuccess) {
+    (void)hipGetLastError();  // not the next launch's
     return 0;
+  }
   return blocks * wpg;
 }
 
