@@ -99,7 +99,7 @@ typedef struct {
                           s.y/y.y of liblbfgs and ncs.cl:1123 */
   int waves_per_group; /* tiles (waves) per workgroup, 1..4; 0 = autotuned
                           (else 4, or 1 for a batch of at most four tiles
-                          per CU) */
+                          per CU that is in device memory) */
   int precision;       /* NCS_PRECISION_* */
 } ncs_params;
 

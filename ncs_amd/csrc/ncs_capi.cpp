@@ -103,9 +103,10 @@ constexpr int kStageSlots = 4;
 constexpr size_t kStageSlot = 1 << 20;
 // Batches up to this many bytes (in and out) are not copied to the device:
 // the solve reads and writes the staging memory over PCIe itself.  Call time
-// with copies and without, us: 64 x 80 67 and 36, 200 x 200 85 and 66,
-// 256 x 256 96 and 93, 300 x 300 109 and 116, 400 x 400 168 and 177,
-// 501 x 643 258 and 226.
+// with copies and without, us, below the limit: 64 x 80 66 and 31, 256 x 256
+// 92 and 65, 400 x 400 164 and 114, 1000 of 16 x 16 223 and 152, 587 x 587 263
+// and 242; above it: 50 of 128 x 128 (6.3 MB) 328 and 324, 700 x 700 (5.6 MB)
+// 316 and 329, 1000 x 1000 520 and 613.
 constexpr size_t kZeroCopyBytes = kStageSlots * kStageSlot;
 
 // A persistent-solve schedule: history depth, grid, workgroup size and the
@@ -728,9 +729,12 @@ static bool any_pad(const ncs_ctx *ctx, const ncs_frame *frames, int n) {
 // 12 against 9 with one; 4 frames of 2048^2 469 against 541 us, 10 frames at
 // history 1 690 against 856 us).  A batch of at most one tile per SIMD leaves
 // the CUs room anyway and starts fastest one wave at a time (30 windows: 16.4
-// against 17.2 us).
-static int default_group(const ncs_ctx *ctx, long long total) {
-  return total <= 4LL * ctx->cus ? 1 : 4;
+// against 17.2 us), but not where it reads the frames over PCIe: neighbouring
+// windows on one CU share what they fetch (call time of a 300 x 300 frame 108
+// us one wave at a time, 81 by fours; 400 x 400 170 and 114, 30 windows 32 and
+// 31).
+static int default_group(const ncs_ctx *ctx, long long total, bool in_place) {
+  return total <= 4LL * ctx->cus && !in_place ? 1 : 4;
 }
 
 // Waves of a schedule's kernel one CU holds at once; 0 where no workgroup fits
@@ -747,14 +751,15 @@ constexpr int kWavesUnknown = 8;
 
 // The schedule of a solve of `total` tiles: explicit params win, then the
 // autotuned schedule of this mask kind and geometry, then history 5,
-// default_group() and the occupancy limit.
+// default_group() and the occupancy limit.  in_place: its frames are in host
+// memory.
 static Schedule resolve_schedule(const ncs_ctx *ctx, const ncs_params *p, bool pad,
-                                 long long total) {
+                                 long long total, bool in_place = false) {
   const bool f16 = p->precision == NCS_PRECISION_F16_SPLIT;
   Schedule d;
   auto it = ctx->tuned.find(TuneKey{ctx->general, pad, f16});
   if (it != ctx->tuned.end()) d = it->second;
-  else d.wpg = default_group(ctx, total);
+  else d.wpg = default_group(ctx, total, in_place);
   Schedule s;
   s.f16 = f16;
   s.history = p->history > 0 ? p->history : d.history;
@@ -829,10 +834,11 @@ static hipError_t launch_schedule(const ncs_ctx *ctx, const Schedule &sc, bool p
 static int enqueue_solve(ncs_ctx *ctx, const FrameDev *d_frames, const FrameDev *inline_frames,
                          int n_frames, bool pad, long long total, const ncs_params *p,
                          const float *u0, int *iters, int *status, float *cost,
-                         unsigned int *queue, hipStream_t s, const Capture &cap = Capture()) {
+                         unsigned int *queue, hipStream_t s, const Capture &cap = Capture(),
+                         bool in_place = false) {
   if (!ctx->has_mask) return fail(NCS_E_NOMASK, "no OTF mask set");
   if (total <= 0) return NCS_OK;
-  const Schedule sc = resolve_schedule(ctx, p, pad, total);
+  const Schedule sc = resolve_schedule(ctx, p, pad, total, in_place);
   SolveArgs a = make_args(ctx, d_frames, n_frames, total, p, u0, iters, status, cost,
                           queue);
   if (queue) {
@@ -1181,7 +1187,8 @@ extern "C" int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int 
       rc = enqueue_solve(ctx, table, fd.data(), n_frames, pad, total, params, nullptr,
                          iterations ? reinterpret_cast<int *>(d_out + r_off[0]) : nullptr,
                          status ? reinterpret_cast<int *>(d_out + r_off[1]) : nullptr,
-                         cost ? reinterpret_cast<float *>(d_out + r_off[2]) : nullptr, nullptr, s);
+                         cost ? reinterpret_cast<float *>(d_out + r_off[2]) : nullptr, nullptr, s,
+                         Capture(), direct);
     if (rc == NCS_OK && !direct) e = download_rows(ctx, out, d_out, out_bytes, s);
     if (rc == NCS_OK && e == hipSuccess) e = mark_solve(ctx, s, Capture());
   }
@@ -1442,7 +1449,7 @@ extern "C" int ncs_hip_autotune(ncs_ctx *ctx, const ncs_frame *frames, int n_fra
   const bool f16 = base->precision == NCS_PRECISION_F16_SPLIT;
   Schedule def;
   def.history = base->history > 0 ? base->history : 5;
-  def.wpg = default_group(ctx, total);
+  def.wpg = default_group(ctx, total, false);
   def.f16 = f16;
   if (occupancy(ctx, def.history, pad, f16, def.wpg) == 0) def.wpg = 1;
   def.waves_per_cu = occupancy(ctx, def.history, pad, f16, def.wpg);
