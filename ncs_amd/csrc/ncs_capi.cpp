@@ -106,7 +106,11 @@ constexpr size_t kStageSlot = 1 << 20;
 // with copies and without, us, below the limit: 64 x 80 66 and 31, 256 x 256
 // 92 and 65, 400 x 400 164 and 114, 1000 of 16 x 16 223 and 152, 587 x 587 263
 // and 242; above it: 50 of 128 x 128 (6.3 MB) 328 and 324, 700 x 700 (5.6 MB)
-// 316 and 329, 1000 x 1000 520 and 613.
+// 316 and 329, 1000 x 1000 520 and 613.  Not where half of them or more are
+// the caller's pinned arrays, which need no copy by the host (see
+// kPinnedBytes): with two of a frame's three arrays pinned 440 x 440 takes 125
+// us read in place and 109 to 125 by DMA, 560 x 560 210 to 214 and 183 to 188;
+// with one 124 and 127 to 131, 214 to 218 and 202 to 219.
 constexpr size_t kZeroCopyBytes = kStageSlots * kStageSlot;
 
 // A persistent-solve schedule: history depth, grid, workgroup size and the
@@ -1058,47 +1062,110 @@ static hipError_t stage_ensure(ncs_ctx *ctx) {
   return r;
 }
 
-// Enqueues the rows' upload to `dst`, slot by slot.  Every slot is free when
-// it starts (each host call waits for the stream before it returns) and its
-// copies may still be running when it returns.
-static hipError_t upload_rows(ncs_ctx *ctx, const std::vector<HostRows> &rows, char *dst,
-                              size_t bytes, hipStream_t s) {
-  RowCursor cur(rows);
+// Arrays of at least this many bytes that the caller has in pinned memory are
+// copied by DMA from and to where they lie; smaller ones are not worth a DMA
+// each.  Call time by DMA and through the slots, us: 20 frames of 351 KB 744
+// and 596, 10 of 511 KB 468 and 457, 10 of 625 KB 521 and 551, one of 4 MB 307
+// and 558, one of 16 MB 1030 and 1943.
+constexpr size_t kPinnedBytes = 512 << 10;
+
+// Whether the rows lie in pinned host memory.
+static bool in_pinned_memory(const HostRows &r) {
+  for (const char *p : {r.p, r.p + (r.n - 1) * r.pitch + r.row - 1}) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+      (void)hipGetLastError();  // memory HIP knows nothing of
+      return false;
+    }
+    if (at.type != hipMemoryTypeHost) return false;
+  }
+  return true;
+}
+
+// How a linear device region's rows travel: the rows in `pinned` by a DMA each
+// to or from byte `at` of the region, the others through the slots, one piece
+// of the region each.  Rows that nobody asked for stay where they are.
+struct RowPlan {
+  struct Piece {
+    size_t at, n;
+  };
+  std::vector<std::pair<size_t, HostRows>> pinned;
+  size_t pinned_bytes = 0;
+  std::vector<HostRows> staged;
+  std::vector<Piece> pieces;
+
+  explicit RowPlan(const std::vector<HostRows> &rows) {
+    size_t at = 0;
+    for (const HostRows &r : rows) {
+      const size_t bytes = r.row * r.n;
+      if (r.p && bytes >= kPinnedBytes && in_pinned_memory(r)) {
+        pinned.emplace_back(at, r);
+        pinned_bytes += bytes;
+      } else if (r.p) {
+        staged.push_back(r);
+        for (size_t o = 0; o < bytes;) {
+          if (pieces.empty() || pieces.back().at + pieces.back().n != at + o ||
+              pieces.back().n == kStageSlot)
+            pieces.push_back({at + o, 0});
+          const size_t n = std::min(kStageSlot - pieces.back().n, bytes - o);
+          pieces.back().n += n;
+          o += n;
+        }
+      }
+      at += bytes;
+    }
+  }
+};
+
+// Enqueues the rows' upload to `dst`, the staged ones slot by slot.  Every slot
+// is free when it starts (each host call waits for the stream before it
+// returns) and its copies may still be running when it returns.
+static hipError_t upload_rows(ncs_ctx *ctx, const RowPlan &plan, char *dst, hipStream_t s) {
   hipError_t e = hipSuccess;
-  int k = 0;
-  for (size_t at = 0; at < bytes && e == hipSuccess; at += kStageSlot, k++) {
-    const int slot = k % kStageSlots;
-    if (k >= kStageSlots) e = hipEventSynchronize(ctx->stage_event[slot]);
+  for (const auto &[at, r] : plan.pinned)
+    if (e == hipSuccess)
+      e = r.n == 1 ? hipMemcpyAsync(dst + at, r.p, r.row, hipMemcpyHostToDevice, s)
+                   : hipMemcpy2DAsync(dst + at, r.row, r.p, r.pitch, r.row, r.n,
+                                      hipMemcpyHostToDevice, s);
+  RowCursor cur(plan.staged);
+  for (size_t k = 0; k < plan.pieces.size() && e == hipSuccess; k++) {
+    const RowPlan::Piece &q = plan.pieces[k];
+    const size_t slot = k % kStageSlots;
+    if (k >= (size_t)kStageSlots) e = hipEventSynchronize(ctx->stage_event[slot]);
     if (e != hipSuccess) break;
     char *buf = ctx->stage + slot * kStageSlot;
-    const size_t n = std::min(kStageSlot, bytes - at);
-    cur.gather(buf, n);
-    e = hipMemcpyAsync(dst + at, buf, n, hipMemcpyHostToDevice, s);
+    cur.gather(buf, q.n);
+    e = hipMemcpyAsync(dst + q.at, buf, q.n, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipEventRecord(ctx->stage_event[slot], s);
   }
   return e;
 }
 
-// Downloads `bytes` from `src` into the rows: the copies run a ring of slots
-// ahead of the host, which returns with every row written.
-static hipError_t download_rows(ncs_ctx *ctx, const std::vector<HostRows> &rows, const char *src,
-                                size_t bytes, hipStream_t s) {
-  RowCursor cur(rows);
-  const size_t pieces = (bytes + kStageSlot - 1) / kStageSlot;
+// Downloads the rows from `src`: the copies run a ring of slots ahead of the
+// host, which returns with every staged row written; the pinned ones are
+// written when the stream is through.
+static hipError_t download_rows(ncs_ctx *ctx, const RowPlan &plan, const char *src,
+                                hipStream_t s) {
+  RowCursor cur(plan.staged);
   hipError_t e = hipSuccess;
-  auto piece = [&](size_t k) { return std::min(kStageSlot, bytes - k * kStageSlot); };
   auto enqueue = [&](size_t k) {
-    const int slot = (int)(k % kStageSlots);
-    hipError_t r = hipMemcpyAsync(ctx->stage + slot * kStageSlot, src + k * kStageSlot, piece(k),
-                                  hipMemcpyDeviceToHost, s);
+    const size_t slot = k % kStageSlots;
+    hipError_t r = hipMemcpyAsync(ctx->stage + slot * kStageSlot, src + plan.pieces[k].at,
+                                  plan.pieces[k].n, hipMemcpyDeviceToHost, s);
     return r == hipSuccess ? hipEventRecord(ctx->stage_event[slot], s) : r;
   };
+  const size_t pieces = plan.pieces.size();
   for (size_t k = 0; k < pieces && k < (size_t)kStageSlots && e == hipSuccess; k++) e = enqueue(k);
+  for (const auto &[at, r] : plan.pinned)
+    if (e == hipSuccess)
+      e = r.n == 1 ? hipMemcpyAsync(r.p, src + at, r.row, hipMemcpyDeviceToHost, s)
+                   : hipMemcpy2DAsync(r.p, r.pitch, src + at, r.row, r.row, r.n,
+                                      hipMemcpyDeviceToHost, s);
   for (size_t k = 0; k < pieces && e == hipSuccess; k++) {
-    const int slot = (int)(k % kStageSlots);
+    const size_t slot = k % kStageSlots;
     e = hipEventSynchronize(ctx->stage_event[slot]);
     if (e != hipSuccess) break;
-    cur.scatter(ctx->stage + slot * kStageSlot, piece(k));
+    cur.scatter(ctx->stage + slot * kStageSlot, plan.pieces[k].n);
     if (k + kStageSlots < pieces) e = enqueue(k + kStageSlots);
   }
   return e;
@@ -1157,7 +1224,10 @@ extern "C" int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int 
     if (results[k]) r_off[k] = add(out, out_bytes, results[k], total * 4ull, total * 4ull, 1);
 
   HIPCHK(stage_ensure(ctx));
-  const bool direct = in_bytes + out_bytes <= kZeroCopyBytes;
+  const RowPlan up(in), down(out);
+  const size_t bytes = in_bytes + out_bytes;
+  const bool direct =
+      bytes <= kZeroCopyBytes && 2 * (up.pinned_bytes + down.pinned_bytes) < bytes;
   char *d_in, *d_out;
   if (direct) {
     void *dev = nullptr;
@@ -1179,7 +1249,7 @@ extern "C" int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int 
   }
   schedule_small_first(fd, total);
   const bool pad = any_pad(ctx, frames, n_frames);
-  hipError_t e = direct ? hipSuccess : upload_rows(ctx, in, d_in, in_bytes, s);
+  hipError_t e = direct ? hipSuccess : upload_rows(ctx, up, d_in, s);
   if (e == hipSuccess) {
     const FrameDev *table = nullptr;
     rc = upload_frames(ctx, fd, s, &table);
@@ -1189,7 +1259,7 @@ extern "C" int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int 
                          status ? reinterpret_cast<int *>(d_out + r_off[1]) : nullptr,
                          cost ? reinterpret_cast<float *>(d_out + r_off[2]) : nullptr, nullptr, s,
                          Capture(), direct);
-    if (rc == NCS_OK && !direct) e = download_rows(ctx, out, d_out, out_bytes, s);
+    if (rc == NCS_OK && !direct) e = download_rows(ctx, down, d_out, s);
     if (rc == NCS_OK && e == hipSuccess) e = mark_solve(ctx, s, Capture());
   }
   // whatever was enqueued is complete before the caller's memory is let go
