@@ -187,9 +187,10 @@ struct ncs_ctx {
   unsigned long long captured_id = 0;
   // device address of the allocation-free entry point's scratch on this GPU
   void *scratch = nullptr;
-  // pinned staging of the host-memory entry points: kStageSlots slots, each
-  // with the event of its last copy
+  // pinned staging of the host-memory entry points: up to kStageSlots slots,
+  // each with the event of its last copy
   char *stage = nullptr;
+  size_t stage_bytes = 0;
   hipEvent_t stage_event[kStageSlots] = {};
   ReplayLine line;
 };
@@ -1049,16 +1050,27 @@ class RowCursor {
   size_t seg_ = 0, row_ = 0, off_ = 0;
 };
 
-static hipError_t stage_ensure(ncs_ctx *ctx) {
-  if (ctx->stage) return hipSuccess;
+// At least `bytes` of staging memory, which is idle between host calls: as
+// much as the context's largest call so far needed, rounded up (a context that
+// solves single windows keeps 64 KB, not the 4 MB of all the slots).
+static hipError_t stage_ensure(ncs_ctx *ctx, size_t bytes) {
+  if (ctx->stage_bytes >= bytes) return hipSuccess;
   for (hipEvent_t &e : ctx->stage_event)
     if (!e) {
       const hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming);
       if (r != hipSuccess) return r;
     }
+  size_t cap = 64 << 10;
+  while (cap < bytes) cap *= 2;
+  if (ctx->stage) (void)hipHostFree(ctx->stage);
+  ctx->stage = nullptr;
+  ctx->stage_bytes = 0;
   void *p = nullptr;
-  const hipError_t r = hipHostMalloc(&p, kStageSlots * kStageSlot, hipHostMallocDefault);
-  if (r == hipSuccess) ctx->stage = static_cast<char *>(p);
+  const hipError_t r = hipHostMalloc(&p, cap, hipHostMallocDefault);
+  if (r == hipSuccess) {
+    ctx->stage = static_cast<char *>(p);
+    ctx->stage_bytes = cap;
+  }
   return r;
 }
 
@@ -1223,11 +1235,13 @@ extern "C" int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int 
   for (int k = 0; k < 3; k++)
     if (results[k]) r_off[k] = add(out, out_bytes, results[k], total * 4ull, total * 4ull, 1);
 
-  HIPCHK(stage_ensure(ctx));
   const RowPlan up(in), down(out);
   const size_t bytes = in_bytes + out_bytes;
   const bool direct =
       bytes <= kZeroCopyBytes && 2 * (up.pinned_bytes + down.pinned_bytes) < bytes;
+  const size_t slots =
+      std::min<size_t>(kStageSlots, std::max(up.pieces.size(), down.pieces.size()));
+  HIPCHK(stage_ensure(ctx, direct ? bytes : slots * kStageSlot));
   char *d_in, *d_out;
   if (direct) {
     void *dev = nullptr;
