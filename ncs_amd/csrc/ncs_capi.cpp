@@ -637,9 +637,10 @@ static int build_frames(const ncs_ctx *ctx, const ncs_frame *frames, int n,
   return describe_frames(ctx, frames, n, fd.data(), total);
 }
 
-// Frame order of the schedule.  The solver claims tiles in frame-table order:
-// the first half in static per-wave blocks, the rest from per-XCD queues, so
-// the last tiles claimed set the launch's tail.  Frames are scheduled smallest
+// Frame order of the schedule.  The solver claims tiles in frame-table order,
+// static per-wave blocks first, then the per-XCD queues where there are any
+// (launch_solve has the shares), so the last tiles claimed set the launch's
+// tail.  Frames are scheduled smallest
 // first (stable, by tile count): small frames and ROIs carry the tiles that
 // run long (edge blocks that are mostly padding, few valid pixels), and this
 // order gives them to many waves at the start, leaving ordinary full tiles of
@@ -730,14 +731,15 @@ static bool any_pad(const ncs_ctx *ctx, const ncs_frame *frames, int n) {
 
 // Waves per workgroup without a tuned schedule.  A workgroup shares one copy
 // of the solver's tables in LDS, which beside the histories decides how many
-// waves a CU holds: four per group hold the most at every depth (history 5:
-// 12 against 9 with one; 4 frames of 2048^2 469 against 541 us, 10 frames at
-// history 1 690 against 856 us).  A batch of at most one tile per SIMD leaves
-// the CUs room anyway and starts fastest one wave at a time (30 windows: 16.4
-// against 17.2 us), but not where it reads the frames over PCIe: neighbouring
-// windows on one CU share what they fetch (call time of a 300 x 300 frame 108
-// us one wave at a time, 81 by fours; 400 x 400 170 and 114, 30 windows 32 and
-// 31).
+// waves a CU holds, and four per group are the fastest or within the noise of it
+// but at history 8 (2048^2, groups of 1, 2, 3 and 4, us: 4 frames, plain start,
+// history 5 584, 394, 383, 374; history 8 591, 532, 501, 533; 10 frames, linear
+// start, history 1 796, 591, 604, 591).  A batch of at most one tile per SIMD
+// leaves the CUs room anyway and starts fastest one wave at a time (30 windows:
+// 16.4 against 17.2 us), but not where it reads the frames over PCIe:
+// neighbouring windows on one CU share what they fetch (call time of a
+// 300 x 300 frame 108 us one wave at a time, 81 by fours; 400 x 400 170 and
+// 114, 30 windows 32 and 31).
 static int default_group(const ncs_ctx *ctx, long long total, bool in_place) {
   return total <= 4LL * ctx->cus && !in_place ? 1 : 4;
 }

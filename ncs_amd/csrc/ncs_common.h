@@ -45,7 +45,7 @@ inline unsigned int div_magic(unsigned int d) {
   if (d <= 1) return 0;
   int l = 0;
   while ((1ull << l) < d) l++;
-  // 2^(31 + l) / d by parts: l <= 31, the quotient is below 2^32
+  // l <= 31, and the quotient is below 2^32
   const unsigned long long p = 1ull << (31 + l);
   return (unsigned int)(p / d + 1);
 }

@@ -699,9 +699,9 @@ __device__ __forceinline__ void grad_w32(const LdsByte *dz, const int (&oz)[2],
 // rows, masked by the ReLU of the activations there, as BF16 in registers:
 // the convolution of dz with the flipped, transposed weights (packs: the
 // lane's entries of the nine taps, read from L2 at each use: kept in
-// registers over the tiles they spilled), each accumulator from zero.  z points
-// at the lane's pixel of padded row 8 h, act at the lane's four channels of
-// row 8 h's pixels (padded).
+// registers over the tiles they spilled), each accumulator from zero.  z
+// points at the lane's pixel of padded row 8 h, act at the lane's four channels
+// of row 8 h's pixels (padded).
 __device__ __forceinline__ void grad_data32(const LdsByte *z, const LdsByte *act,
                                             const i4 *__restrict__ packs, i2v (&out)[8]) {
   i4 A[9];

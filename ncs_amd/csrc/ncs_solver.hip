@@ -1636,7 +1636,8 @@ hipError_t launch_eval(bool general, const float *data, const float *gamma, cons
   return hipGetLastError();
 }
 
-// Half tiles per wave (4.5 tiles) up to which a launch is all static.
+// Half tiles per wave (4.5 tiles) up to which a launch is all static (see
+// launch_solve).
 constexpr long long kStaticHalfTiles = 9;
 
 // Resets the work-queue counters (a kernel, not a memset, so that captured
@@ -1704,10 +1705,14 @@ int solve_waves_per_cu(int m, bool general, bool pad, bool f16, int wpg) {
 // 4.5 tiles per wave all of them (each SIMD's handful of waves ends
 // with the same number of tiles give or take one, and the launch needs no
 // counters; one tile per wave is the smallest batch's best: 30 windows went
-// from 55 us, in chunks on eight waves, to 16 us).  Above that two fifths,
-// and the rest one by one, which evens out the waves: with history 1 and the
-// linear start, 10 frames of 2048^2 take 704 us at one half static in chunks
-// of four, 671 us as here (664 at one quarter, 722 at four fifths); with
+// from 55 us, in chunks on eight waves, to 16 us).  4.5 lies between the two
+// starts' crossings.  All static and with the dynamic share, one frame, us:
+// plain start, history 5 (its tiles differ more), 2.4 tiles a wave 59 and 64,
+// 3.2 76 and 72, 4.5 100 and 94, 5.3 118 and 108; linear start, history 1, 2.6
+// 50 and 57, 4.2 76 and 84, 5.3 93 and 97, 7.8 134 and 129.  Above that two
+// fifths, and the rest one by one, which evens out the waves: with history 1
+// and the linear start, 10 frames of 2048^2 take 704 us at one half static in
+// chunks of four, 671 us as here (664 at one quarter, 722 at four fifths); with
 // history 5 and the plain start 1095 and 1084 us (1087, 1140); one frame
 // 120 and 87 us, 150 and 128 us.  Chunks of two or three were within 1% with
 // the linear start's short tiles and 2% slower with the plain start's.
