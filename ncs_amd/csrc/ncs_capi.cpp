@@ -125,14 +125,15 @@ struct Schedule {
 // Key of an autotuned schedule: mask kind, padded geometry, precision.
 typedef std::array<bool, 3> TuneKey;
 
-// The last replay whose download took its turn on the PCIe link (see
-// takes_turns): its pipeline and the event behind it.  The pipelines of a
-// context share it, each from its own thread if need be; a pipeline takes
-// itself out before its events go.
+// Replays that take turns on the PCIe link (see takes_turn): the pipelines
+// that may, the one of them that was launched last, and the streams that such
+// replays' uploads, graphs and downloads go through.  The pipelines of a
+// context share it, each from its own thread if need be.
 struct ReplayLine {
   std::mutex mu;
-  const ncs_pipeline *owner = nullptr;
-  hipEvent_t done = nullptr;
+  std::vector<const ncs_pipeline *> members;
+  const ncs_pipeline *last = nullptr;
+  hipStream_t up = nullptr, solve = nullptr, down = nullptr;
 };
 
 struct ncs_ctx {
@@ -349,6 +350,8 @@ extern "C" void ncs_hip_destroy(ncs_ctx *ctx) {
   DevBuf *bufs[] = {&ctx->tables, &ctx->frames, &ctx->queue, &ctx->in, &ctx->out,
                     &ctx->net_params, &ctx->net_packs, &ctx->net_tmp_packs, &ctx->u0_buf};
   for (DevBuf *b : bufs) b->release();
+  for (hipStream_t s : {ctx->line.up, ctx->line.solve, ctx->line.down})
+    if (s) (void)hipStreamDestroy(s);
   if (ctx->frames_event) (void)hipEventDestroy(ctx->frames_event);
   for (hipEvent_t ev : {ctx->solve_done, ctx->captured_done})
     if (ev) (void)hipEventDestroy(ev);
@@ -1644,6 +1647,7 @@ struct ncs_pipeline {
   std::vector<char> gamma_set;
   hipStream_t stream = nullptr;
   hipEvent_t done[kReplaySlots] = {};
+  hipEvent_t uploaded = nullptr, solved = nullptr;  // of a replay that takes its turn
   long long launched = 0;  // replays enqueued
   long long waited = 0;    // replays known to be complete
   hipStream_t last_stream = nullptr;
@@ -1652,12 +1656,72 @@ struct ncs_pipeline {
   std::vector<float *> cur_out;
 };
 
+// Replays of like pipelines take turns on the PCIe link: the uploads of one
+// follow those of the other pipeline's replay before it, and so do the
+// downloads.  Left alone, two of them share the link each way: neither has its
+// image before both are nearly through, and the link then idles for the next
+// upload and solve.  They go through three streams of the context's, one each
+// for uploads, graphs and downloads.  Six 2304 x 2304 frames through two
+// pipelines take 2790 us instead of 3360 to 3540 (16-bit input) and 3295
+// instead of 3980 to 4440 (FP32).
+// Only where that pays and cannot cost:
+//  * another pipeline does the same work, so the one enqueued first is ready
+//    first, and it, or none, was launched last (a pipeline that runs alone
+//    would pay some 7 us a replay for the hand-overs);
+//  * the replay is the pipeline's only one under way and not on a caller's
+//    stream, so its buffers are idle and what it waits for is under way;
+//  * the images are large.  Six frames with turns and without, us: 16-bit input
+//    724 x 724 540 and 402 to 533, 1024 x 1024 719 to 788 and 689 to 836, 1300 x
+//    1300 (6.8 MB) 1000 and 1079 to 1217; FP32 545 to 605 and 454 to 553, 818 and
+//    843 to 908, 1185 and 1341 to 1442.
+// The hand-overs stay off the pipelines' own streams because HIP deals a
+// process's streams out to four hardware queues: a wait ahead of an upload
+// stood behind the other pipeline's solve where the two shared a queue, and the
+// six frames took 4235 and 5280 us.
+constexpr size_t kTurnBytes = 6 << 20;
+
+// Puts pl among its context's pipelines that may take turns, if it may.  The
+// streams are made with the first one, one after the other, which gives them
+// hardware queues of their own.
+static hipError_t join_line(ncs_pipeline *pl) {
+  if (pl->pix * sizeof(float) < kTurnBytes) return hipSuccess;
+  ReplayLine &line = pl->ctx->line;
+  std::lock_guard<std::mutex> lk(line.mu);
+  hipError_t e = hipSuccess;
+  for (hipEvent_t *ev : {&pl->uploaded, &pl->solved})
+    if (e == hipSuccess) e = hipEventCreateWithFlags(ev, hipEventDisableTiming);
+  for (hipStream_t *s : {&line.up, &line.solve, &line.down})
+    if (e == hipSuccess && !*s) e = hipStreamCreateWithFlags(s, hipStreamNonBlocking);
+  if (e == hipSuccess) line.members.push_back(pl);
+  return e;
+}
+
+static void leave_line(const ncs_pipeline *pl) {
+  ReplayLine &line = pl->ctx->line;
+  std::lock_guard<std::mutex> lk(line.mu);
+  line.members.erase(std::remove(line.members.begin(), line.members.end(), pl),
+                     line.members.end());
+  if (line.last == pl) line.last = nullptr;
+}
+
+// Whether the replay that pl launches now takes its turn.
+static bool takes_turn(const ncs_pipeline *pl, hipStream_t stream) {
+  if (stream || pl->launched != pl->waited || !pl->solved) return false;
+  ReplayLine &line = pl->ctx->line;
+  std::lock_guard<std::mutex> lk(line.mu);
+  const bool alone = line.last == pl;
+  line.last = pl;
+  return !alone && std::any_of(line.members.begin(), line.members.end(),
+                               [&](const ncs_pipeline *q) {
+                                 return q != pl && q->work == pl->work;
+                               });
+}
+
 extern "C" void ncs_hip_pipeline_destroy(ncs_pipeline *pl) {
   if (!pl) return;
   if (pl->ctx) {
     (void)hipSetDevice(pl->ctx->device);
-    std::lock_guard<std::mutex> lk(pl->ctx->line.mu);
-    if (pl->ctx->line.owner == pl) pl->ctx->line.owner = nullptr;
+    leave_line(pl);
   }
   if (pl->launched > pl->waited)
     (void)hipEventSynchronize(pl->done[(pl->launched - 1) % kReplaySlots]);
@@ -1670,6 +1734,8 @@ extern "C" void ncs_hip_pipeline_destroy(ncs_pipeline *pl) {
     if (pl->h_res[k]) (void)hipHostFree(pl->h_res[k]);
     if (pl->done[k]) (void)hipEventDestroy(pl->done[k]);
   }
+  for (hipEvent_t ev : {pl->uploaded, pl->solved})
+    if (ev) (void)hipEventDestroy(ev);
   if (pl->stream) (void)hipStreamDestroy(pl->stream);
   delete pl;
 }
@@ -1768,6 +1834,7 @@ extern "C" int ncs_hip_pipeline_create(ncs_ctx *ctx, const ncs_pipeline_frame *f
   pl->level_points.resize(n_frames);
   pl->sched = resolve_schedule(ctx, params, pl->pad, pl->total);
   pl->win = ctx->win;
+  HIPCHK(join_line(pl.get()));
   *out = pl.release();
   return NCS_OK;
 }
@@ -1947,53 +2014,33 @@ static int build_pipeline_graph(ncs_pipeline *pl) {
   return NCS_OK;
 }
 
-// Downloads of like pipelines take turns on the PCIe link: a replay's waits
-// for that of the other pipeline's replay before it.  Left alone, two of them
-// share the link: neither has its image before both are nearly through, and
-// the link then idles for the next upload and solve.  Six 2304 x 2304 frames
-// through two pipelines take 3031 us instead of 3285 (16-bit input) and 3719
-// instead of 4429 (FP32).
-// Only where the wait pays and cannot cost:
-//  * both run on their pipelines' own streams with no replay before them that
-//    the caller has not waited for, so what is waited for is under way;
-//  * both do the same work, so the one enqueued first is ready first;
-//  * the images are large: the wait costs the link some 10 us a replay.
-// Uploads do not take turns.  That gained more (2894 and 3417 us), but HIP
-// deals a process's streams out to four hardware queues, and where the two
-// pipelines' share one the wait ahead of an upload stood behind the other's
-// solve, so that nothing overlapped: 4640 and 5650 us.  There the downloads'
-// turns make 3814 us of 3741 and 4234 of 4162.
-constexpr size_t kTurnBytes = 8 << 20;
-
-static bool takes_turns(const ncs_pipeline *pl, hipStream_t stream) {
-  return !stream && pl->launched == pl->waited && pl->pix * sizeof(float) >= kTurnBytes;
+static hipError_t hand_over(hipEvent_t ev, hipStream_t from, hipStream_t to) {
+  const hipError_t e = hipEventRecord(ev, from);
+  return e == hipSuccess ? hipStreamWaitEvent(to, ev, 0) : e;
 }
 
-// Makes s wait for the replay in the line, if another, like pipeline's.
-static hipError_t await_turn(const ncs_pipeline *pl, hipStream_t s) {
-  ReplayLine &line = pl->ctx->line;
-  std::lock_guard<std::mutex> lk(line.mu);
-  if (!line.owner || line.owner == pl || line.owner->work != pl->work) return hipSuccess;
-  return hipStreamWaitEvent(s, line.done, 0);
-}
-
-// Enqueues one replay on s: upload of every frame, the graph, download of
-// every frame and of the per-tile results into the replay's slot.
-static hipError_t enqueue_replay(ncs_pipeline *pl, hipStream_t s, int slot, bool in_turn) {
+// Enqueues one replay: upload of every frame on `up`, the graph on `solve`,
+// download of every frame and of the per-tile results into the replay's slot on
+// `down` (one stream, or the line's three).
+static hipError_t enqueue_replay(ncs_pipeline *pl, hipStream_t up, hipStream_t solve,
+                                 hipStream_t down, int slot) {
   char *dev_in = pl->input == NCS_INPUT_ADU_U16 ? pl->raw.as<char>() : pl->data.as<char>();
   hipError_t e = hipSuccess;
   for (int i = 0; i < pl->n && e == hipSuccess; i++)
     e = hipMemcpyAsync(dev_in + pl->off[i] * pl->elem, pl->cur_in[i],
-                       frame_pixels(pl->shape[i]) * pl->elem, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipGraphLaunch(pl->exec, s);
-  if (e == hipSuccess && in_turn) e = await_turn(pl, s);
+                       frame_pixels(pl->shape[i]) * pl->elem, hipMemcpyHostToDevice, up);
+  if (e == hipSuccess && up != solve) e = hand_over(pl->uploaded, up, solve);
+  if (e == hipSuccess) e = hipGraphLaunch(pl->exec, solve);
+  if (e == hipSuccess && solve != down) e = hand_over(pl->solved, solve, down);
   for (int i = 0; i < pl->n && e == hipSuccess; i++)
     e = hipMemcpyAsync(pl->cur_out[i], pl->out.as<float>() + pl->off[i],
-                       frame_pixels(pl->shape[i]) * sizeof(float), hipMemcpyDeviceToHost, s);
+                       frame_pixels(pl->shape[i]) * sizeof(float), hipMemcpyDeviceToHost, down);
   if (e == hipSuccess && pl->keep) {
     e = hipMemcpyAsync(pl->h_res[slot], pl->results.p, (size_t)pl->total * 12,
-                       hipMemcpyDeviceToHost, s);
+                       hipMemcpyDeviceToHost, down);
   }
+  if (e != hipSuccess && up != down)  // `down` may not be behind what was enqueued
+    for (hipStream_t s : {up, solve}) (void)hipStreamSynchronize(s);
   return e;
 }
 
@@ -2033,24 +2080,20 @@ extern "C" int ncs_hip_pipeline_launch(ncs_pipeline *pl, const void *const *inpu
   }
   if (inputs) pl->cur_in.assign(inputs, inputs + pl->n);
   if (outputs) pl->cur_out.assign(outputs, outputs + pl->n);
-  hipStream_t s = stream ? (hipStream_t)stream : pl->stream;
+  hipStream_t up = stream ? (hipStream_t)stream : pl->stream, solve = up, s = up;
+  if (takes_turn(pl, (hipStream_t)stream))
+    up = ctx->line.up, solve = ctx->line.solve, s = ctx->line.down;
   hipError_t e = hipSuccess;
   // the device buffers are shared by every replay: one enqueued on another
   // stream waits on the device for the previous one
   if (seq > pl->waited && s != pl->last_stream)
     e = hipStreamWaitEvent(s, pl->done[(seq - 1) % kReplaySlots], 0);
-  const bool in_turn = takes_turns(pl, (hipStream_t)stream);
-  if (e == hipSuccess) e = enqueue_replay(pl, s, slot, in_turn);
+  if (e == hipSuccess) e = enqueue_replay(pl, up, solve, s, slot);
   // whatever was enqueued is covered by the replay's event
   hipError_t e2 = hipEventRecord(pl->done[slot], s);
   if (e2 == hipSuccess) {
     pl->launched = seq + 1;
     pl->last_stream = s;
-    if (in_turn && e == hipSuccess) {
-      std::lock_guard<std::mutex> lk(ctx->line.mu);
-      ctx->line.owner = pl;
-      ctx->line.done = pl->done[slot];
-    }
   }
   HIPCHK(e);
   HIPCHK(e2);
