@@ -195,8 +195,8 @@ __device__ __forceinline__ i2v relu_masked(f4 v, i2v act) {
 // lane group next to it (the row swap trades the second half of an even group
 // for the first half of the odd one), every lane has eight channels in a row,
 // 16 (g & 1) + 8 (g >> 1).., and a wave's store is one stretch of 1 KB
-// (8000 tiles, 393 MB of activations: 108.6 -> 101.4 us, with the next tile's
-// inputs loaded under layer 4; two stores of 8 bytes a lane before).
+// (8000 tiles, 393 MB of activations: 108 -> 96 us; two stores of 8 bytes a lane
+// before).
 __device__ __forceinline__ void store_row_std(__bf16 *dst, int y, int lane, i4 v) {
   const int x = lane & 15, g = lane >> 4;
   const auto a = __builtin_amdgcn_permlane16_swap((unsigned int)v.x, (unsigned int)v.z, false,
@@ -464,7 +464,13 @@ __device__ __forceinline__ void stage_forward(const i4 *__restrict__ packs,
 }
 
 // Training / tensor mode: x [n][2][256] normalised inputs -> y [n][256].
-// One wave per tile, its activations in registers.
+// One wave per tile, its activations in registers; KEEP: written to acts too.
+// A tile's inputs are loaded where they are used.  Loaded under the layer 4
+// before (as the kernel over frames does) they spilled 13 registers of a build
+// for both kinds, which took longer than what it hid: 8000 tiles with
+// activations 97 us, 85 now; without 53 and 48; 2048 without 18.6 and 15.8
+// (17.4 before the loads were moved).
+template <bool KEEP>
 __global__ __launch_bounds__(64 * kNetWaves) __attribute__((amdgpu_waves_per_eu(2)))
 void net_fwd_kernel(const float *__restrict__ xin, float *__restrict__ yout,
                     __bf16 *__restrict__ acts, const i4 *__restrict__ packs,
@@ -478,26 +484,20 @@ void net_fwd_kernel(const float *__restrict__ xin, float *__restrict__ yout,
   int *const grid = reinterpret_cast<int *>(bl + 128 + wave * kNetWaveFloats);
   float *const dbuf = reinterpret_cast<float *>(grid + kNetGridInts);
   const int col = lane & 15, grp = lane >> 4;
-  float x0[4], x1[4];
-  auto load = [&](long long t) {
+  stage_forward(packs, P, pk, bl);
+  in_pad_border(grid, lane);
+  for (long long t = (long long)blockIdx.x * kNetWaves + wave; t < n;
+       t += (long long)gridDim.x * kNetWaves) {
     const float *const x = xin + t * 512;
+    float x0[4], x1[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
       x0[k] = x[lane + 64 * k];
       x1[k] = x[lane + 64 * k + 256];
     }
-  };
-  const long long stride = (long long)gridDim.x * kNetWaves;
-  long long t = (long long)blockIdx.x * kNetWaves + wave;
-  if (t < n) load(t);
-  stage_forward(packs, P, pk, bl);
-  in_pad_border(grid, lane);
-  for (; t < n; t += stride) {
 #pragma unroll
     for (int k = 0; k < 4; k++) in_pad_put(grid, 4 * k + grp, col, x0[k], x1[k]);
-    const f4 y = net_body(grid, dbuf, pk, bl, lane, acts, n, t, [&] {
-      if (t + stride < n) load(t + stride);
-    });
+    const f4 y = net_body(grid, dbuf, pk, bl, lane, KEEP ? acts : nullptr, n, t, [] {});
 #pragma unroll
     for (int r = 0; r < 4; r++) yout[t * 256 + (4 * grp + r) * 16 + col] = y[r];
     wave_sync();
@@ -1098,7 +1098,8 @@ int net_forward_grid(long long n, int cus) {
 hipError_t net_forward(const float *x, float *y, void *acts, const void *packs, const float *P,
                        long long n, int grid, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(net_fwd_kernel, dim3(grid), dim3(64 * kNetWaves), kNetFwdLdsBytes, s, x, y,
+  hipLaunchKernelGGL(acts != nullptr ? net_fwd_kernel<true> : net_fwd_kernel<false>, dim3(grid),
+                     dim3(64 * kNetWaves), kNetFwdLdsBytes, s, x, y,
                      reinterpret_cast<__bf16 *>(acts), reinterpret_cast<const i4 *>(packs), P, n);
   return hipGetLastError();
 }
