@@ -572,12 +572,18 @@ void net_warm_kernel(WithFrames<NetWarmArgs> W) {
   // The two waves of a SIMD start together and run the same tile in the same
   // time: both would convert, shift and wait in step, with the matrix cores
   // idle.  Each is favoured on every other tile, which keeps them apart (two
-  // 2048^2 frames, net and solve: 424 -> 418 us; always the same one: 427).
+  // 2048^2 frames, net and solve: 424 -> 418 us; always the same one: 427).  Up
+  // to one and a half tiles a wave the other one would end alone: 2116 tiles on
+  // 2048 waves 23.7 us so and 21.7 without, 3025 23.9 and 22.1; 3249 26.0 and
+  // 28.0.
+  const bool apart = 2 * total > 3 * stride;
   bool favoured = 2 * blockIdx.x >= gridDim.x;
   for (; t < total; t += stride) {
-    if (favoured) __builtin_amdgcn_s_setprio(1);
-    else __builtin_amdgcn_s_setprio(0);
-    favoured = !favoured;
+    if (apart) {
+      if (favoured) __builtin_amdgcn_s_setprio(1);
+      else __builtin_amdgcn_s_setprio(0);
+      favoured = !favoured;
+    }
     float sigma;
     tile_inputs(d, gm, grid, lane, sigma);
 #pragma unroll
