@@ -161,7 +161,9 @@ long long ncs_hip_tile_count_window(int height, int width, int geometry, int r);
  * entry per tile, frames in order, tiles in raster order.  The launch
  * schedules the frames smallest first (stable, by tile count), so that the
  * long-running tiles of small frames and ROIs start early; results and the
- * order of every per-tile array are the same as in the caller's order. */
+ * order of every per-tile array are the same as in the caller's order.  Arrays
+ * of 512 KB and more in pinned memory (hipHostMalloc) are copied by DMA from
+ * and to where they lie, others through pinned memory of the context's. */
 int ncs_hip_reduce_frames(ncs_ctx *ctx, const ncs_frame *frames, int n_frames,
                           const ncs_params *params, int *iterations,
                           int *status, float *cost);
